@@ -5,16 +5,15 @@
 // HBM layout:
 //   * captured signals It, dIt/dv, dIt/dvpre are time-major (T, N) fp32, T =
 //     ksteps + 1, row 0 zero: a capture writes one contiguous row per LR tick;
-//   * dense block b (bn x bn x K_len, the caller's kernel K_b[i][j][tau]) is
-//     kept twice, tau-major: kt1 = K_b[i][j][tau] at [tau][i][j] (base term) and
-//     kt2 = K_b[j][k][tau] at [tau][k][j] (the correction GEMM's B operand,
-//     contiguous in the output column j);
-//   * the dv/dw history is a ring of K_len + 1 row-major N x N fp32 slices:
-//     tick tau lives in slot tau % (K_len + 1), slot 0 starts as the zero slice
-//     of tick 0, and the slot a tick writes is never in its own read window.
-//     A second ring holds each slice's column-gathered copy G[i][c] =
-//     D[i][pre(c)], written once per tick, so the correction's pre operand is a
-//     contiguous read instead of a gather per (row, tap);
+//   * dense block b (bn x bn x K_len, the caller's kernel K_b[i][j][tau]) is kept
+//     tau-major at [tau][i][j], rows padded with zeros to bnp = bn rounded up to 4: the
+//     base term reads K_b[i][j][tau], and as K_b[j][k][tau] the same array is the
+//     correction GEMM's second operand, contiguous in the reduction index k;
+//   * the history is a ring of K_len + 1 slices X_tau, the correction's first operand:
+//     block after block, each N rows of bnp floats (the padding zero, never written).
+//     Tick tau lives in slot tau % (K_len + 1), slot 0 starts as tick 0's, and the slot a
+//     tick writes is never in its own read window.  The dv/dw slices alternate between
+//     two buffers (the previous one is still read for dx).
 //     A per-slot fp32 scale carries the Frobenius clip's rescaling of the history
 //     instead of rewriting K_len slices.
 #pragma once
@@ -26,8 +25,13 @@
 namespace hx {
 
 constexpr int kLrMaxChannels = 3;     // pure_i, didv, didvpre
-// Size of the per-device scratch array of the allocation-free replay (64 MiB).
-constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(64) << 20;
+// The allocation-free replay: problems of at most kNoAllocLimitBytes of signals, slices
+// and vectors (16 N T + 8 R N^2 bytes and the small ones) are taken; the per-device scratch
+// array holds what the kernels need for any of those (block rows padded to multiples of 4,
+// the correction's split sums).
+constexpr size_t kNoAllocLimitBytes = static_cast<size_t>(64) << 20;
+constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(256) << 20;
+constexpr int kBaseTicks = 8;         // ticks whose base terms one launch makes
 
 struct CaptureChannel {
     const int* begin = nullptr;       // N + 1: items of column c are [begin[c], begin[c+1])
@@ -46,57 +50,112 @@ struct CaptureArgs {
 };
 
 struct ReplayBaseArgs {
-    const float* kt1 = nullptr;
-    const long long* koff = nullptr;  // per block offset into kt1 / kt2
+    const float* kp = nullptr;
+    const long long* koff = nullptr;  // per block offset into kp
     const long long* boff = nullptr;  // per block offset into base (sum of bn^2)
     const int* start = nullptr;
     const int* bn = nullptr;
+    const int* bnp = nullptr;
     const float* it = nullptr;        // (T, N)
-    int N = 0, it_t0 = 0, k_t0 = 0, tw = 0;
+    int N = 0, T = 0, K_len = 0;
+    int t0 = 0, ng = 0;               // ticks t0 .. t0 + ng - 1
+    float* base = nullptr;            // tap sums, one set of base_stride floats per tick
+    long long base_stride = 0;
+};
+
+// dx of one finished tick (n_in 0: none)
+struct ReplayDx {
+    const float* cur = nullptr;       // the tick's slice
+    const int* pin = nullptr;
+    int n_in = 0;
+    const float* w_tick = nullptr;
+    float eps = 0.f;
+    int t_idx = 0, ksteps = 0;
+    int clip_ran = 0;
+    const float* tick_scale = nullptr;
+    float* dx = nullptr;
+};
+
+// where a tick's slice goes and what is added to its correction
+struct ReplayOut {
+    int N = 0;
     float dt = 0.f;
     const float* gs = nullptr;        // device grad scale
-    float* base = nullptr;
-    float* slot_scale = nullptr;      // slot_scale[cur] is reset to 1
-    int cur = 0;
+    const float* base = nullptr;      // this tick's tap sums
+    float* out = nullptr;
+    int sanitize = 0;                 // zero non-finite entries and write norm partials
+    double* norm_part = nullptr;
 };
 
 struct ReplayCorrArgs {
-    const float* hist = nullptr;
-    const float* ghist = nullptr;     // column-gathered copies: ghist[h][i][c] = hist[h][i][pre(c)]
-    long long slice = 0;              // N * N
+    const float* x = nullptr;         // the ring of X slices
+    long long xslice = 0;             // floats per slice
+    const long long* xoff = nullptr;  // per block offset into a slice
     const float* slot_scale = nullptr;
     int R = 1;                        // ring slots
-    const float* dv = nullptr;        // dIt/dv (T, N)
-    const float* dp = nullptr;        // dIt/dvpre (T, N)
-    const int* pre = nullptr;
-    const float* kt2 = nullptr;
+    int h0 = 0;                       // slot of the window's first tick
+    const float* kp = nullptr;
     const long long* koff = nullptr;
     const int* start = nullptr;
     const int* bn = nullptr;
-    const float* base = nullptr;
+    const int* bnp = nullptr;
     const long long* boff = nullptr;
     const int2* tiles = nullptr;      // (block, first column) of each column tile
-    int N = 0, t_lr = 0, tw = 0, it_t0 = 0, k_t0 = 0;
-    float dt = 0.f;
-    float* out = nullptr;             // slot of this tick
-    int sanitize = 0;                 // zero non-finite entries and write norm partials
-    double* norm_part = nullptr;
-    int* flag_part = nullptr;
+    int row_tiles = 0, nsplit = 1, ncorr = 0;   // ncorr: column tiles x row tiles x splits
+    int tw = 0, k_t0 = 0;
+    float* part = nullptr;            // nsplit > 1: the splits' sums, N x N each
+    ReplayOut O;
+    ReplayDx dx;
+};
+
+struct ReplayFinishArgs {
+    const float* part = nullptr;
+    int nsplit = 0;                   // 0: no correction
+    int nblock = 0;                   // set by the launcher
+    const int* col_block = nullptr;   // block of each column
+    const int* start = nullptr;
+    const int* bn = nullptr;
+    const long long* boff = nullptr;
+    ReplayOut O;
+    ReplayDx dx;
+};
+
+struct ReplayTickArgs {
+    int N = 0;
+    const float* cur = nullptr;       // the tick's slice
+    int wblocks = 0;                  // set by the launcher
+    int due = 0;                      // clip tick
+    const double* norm_part = nullptr;
+    int npart = 0;
+    float thr = 0.f;
+    float* gs = nullptr;
+    float* slot_scale = nullptr;
+    int R = 1, cur_slot = 0;
+    float* tick_scale = nullptr;
+    const int* po = nullptr;
+    int n_out = 0;
+    const float* dl = nullptr;        // null: only X
+    float* w_tick = nullptr;
+    float* dw_acc = nullptr;
+    float* x = nullptr;               // slot of this tick (null: no X)
+    const long long* xoff = nullptr;
+    const int* col_block = nullptr;
+    const int* start = nullptr;
+    const int* bnp = nullptr;
+    const int* pre = nullptr;
+    const float* dv = nullptr;        // dIt/dv and dIt/dvpre at the next signal time
+    const float* dp = nullptr;
 };
 
 void launch_lr_capture(const CaptureArgs& a, int sample, int lr, hipStream_t s);
 void launch_rp_base(const ReplayBaseArgs& a, int nblk, int max_bn, hipStream_t s);
-void launch_rp_corr(const ReplayCorrArgs& a, int ntiles, int tile_cols, hipStream_t s);
-void launch_rp_pregather(const float* D, const int* pre, int N, float* G, hipStream_t s);
+void launch_rp_corr(const ReplayCorrArgs& a, int tile_cols, hipStream_t s);
 int rp_corr_row_tiles(int N);
-void launch_rp_clip(const double* part, const int* flag, int n, float thr, float* gs, float* slot_scale, int R,
-                    float* tick_scale, hipStream_t s);
-void launch_rp_wtick(const float* cur, const float* slot_scale, int cur_slot, int N, const int* po, int n_out,
-                     const float* dl, int clip_ran, const float* tick_scale, float* w_tick, float* dw_acc,
-                     hipStream_t s);
-void launch_rp_dx(const float* cur, const float* slot_scale, int cur_slot, int N, const int* pin, int n_in,
-                  const float* w_tick, float eps, int t_idx, int ksteps, int clip_ran, const float* tick_scale,
-                  float* dx, hipStream_t s);
+int rp_corr_splits(int N, int ntiles, int max_bnp, int tw);
+void launch_rp_finish(ReplayFinishArgs a, hipStream_t s);
+int rp_finish_blocks(int N);
+void launch_rp_tick(ReplayTickArgs a, hipStream_t s);
+void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s);
 void launch_rp_scale_into(const float* src, float scale, float* dst, long long n, hipStream_t s);
 void launch_fill_f32(float* p, float v, long long n, hipStream_t s);
 void launch_transpose_nt_tn(const float* src_nt, float* dst_tn, int N, int T, hipStream_t s);
@@ -168,10 +227,12 @@ public:
     long long corr_launches = 0;
 
     struct Workspace {
-        float *hist = nullptr, *ghist = nullptr, *slot_scale = nullptr, *gs = nullptr, *tick_scale = nullptr,
-              *w_tick = nullptr, *dw_acc = nullptr, *dl = nullptr, *dx = nullptr, *dw_out = nullptr;
-        int *po = nullptr, *pre = nullptr, *pin = nullptr, *flag_part = nullptr;
+        float *slices = nullptr, *x = nullptr, *part = nullptr, *base = nullptr, *slot_scale = nullptr, *gs = nullptr,
+              *tick_scale = nullptr, *w_tick = nullptr, *dw_acc = nullptr, *dl = nullptr, *dx = nullptr,
+              *dw_out = nullptr;
+        int *po = nullptr, *pre = nullptr, *pin = nullptr;
         double* norm_part = nullptr;
+        int base_ticks = 0;               // ticks base holds
     };
 
 private:
@@ -180,15 +241,24 @@ private:
     int replay_on(const ReplayIn& in, const Workspace& ws, float* const* sig, int N);
 
     hipStream_t stream_;
+    // Buffer sizes of a replay with and without the precise term, in one place for both
+    // ways of providing them.
+    struct Sizes {
+        int R = 1;
+        size_t x = 0, part = 0, norm = 0;
+    };
+    Sizes sizes_for(int N, bool percise) const;
+
     // dense blocks
-    int k_len_ = 0, nblk_ = 0, max_bn_ = 0, tile_cols_ = 64;
+    int k_len_ = 0, nblk_ = 0, max_bn_ = 0, max_bnp_ = 0, tile_cols_ = 64;
     std::vector<int> bn_, start_;
-    std::vector<long long> koff_, boff_;
+    std::vector<long long> koff_, boff_, xoff_;
+    long long base_len_ = 0, xcols_ = 0;    // sum of bn^2, sum of bnp
     std::vector<int2> tiles_;
     std::vector<void*> blk_mem_;
-    float *d_kt1_ = nullptr, *d_kt2_ = nullptr, *d_base_ = nullptr;
-    long long *d_koff_ = nullptr, *d_boff_ = nullptr;
-    int *d_start_ = nullptr, *d_bn_ = nullptr;
+    float* d_kp_ = nullptr;
+    long long *d_koff_ = nullptr, *d_boff_ = nullptr, *d_xoff_ = nullptr;
+    int *d_start_ = nullptr, *d_bn_ = nullptr, *d_bnp_ = nullptr, *d_col_block_ = nullptr;
     int2* d_tiles_ = nullptr;
     // capture cache (T, N) per channel
     int cap_N_ = 0, cap_T_ = 0, cap_kmul_ = 0;
@@ -206,6 +276,9 @@ private:
     std::vector<void*> sess_mem_;
     // host-loaded signals (T, N)
     int sig_N_ = 0, sig_T_ = 0;
+    size_t sig_cap_ = 0;                // floats each signal buffer holds
+    int sig_ch_ = 0;                    // signal buffers there are
+    float* d_sig_stage_ = nullptr;
     std::vector<void*> sig_mem_;
     float* d_sig_[kLrMaxChannels] = {nullptr, nullptr, nullptr};
     // replay workspace, kept while the problem shape is unchanged

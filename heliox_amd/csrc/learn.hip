@@ -6,16 +6,18 @@
 // t, kernel taps k_t0 = K_len - tw ... K_len - 1) the replay forms
 //
 //   dvtdw_t[i, s+j] = [i in block] (sum_u K_b[i-s][j][k_t0+u] It[it_t0+u][i]) dt gs
-//                   + dt sum_{u,k} K_b[j][k][k_t0+u] X_u[i, k]
-//   X_u[i, k] = dvtdw_{t-tw+u}[i, s+k] dIt/dv[it_t0+u][s+k]
-//             + dvtdw_{t-tw+u}[i, pre(s+k)] dIt/dvpre[it_t0+u][s+k]
+//                   + dt sum_{u,k} K_b[j][k][k_t0+u] X_{t-tw+u}[i, k]
+//   X_tau[i, k] = dvtdw_tau[i, s+k] dIt/dv[tau+1][s+k]
+//               + dvtdw_tau[i, pre(s+k)] dIt/dvpre[tau+1][s+k]
 //
-// (base term replay_dw_dx.cu:227-274, correction :282-325).  The correction is
-// a GEMM per block, (N x bn*tw) X times (bn*tw x bn) K: k_rp_corr computes it
-// with v_mfma_f32_32x32x2f32, forming X on the fly from the history slices as
-// it stages each 128-row x 32-tap chunk through LDS.  The pre(s+k) operand is
-// read from a column-gathered copy of each slice made once when the slice is
-// written (k_rp_pregather), so every history read is a contiguous row segment.
+// (base term replay_dw_dx.cu:227-274, correction :282-325).  X_tau depends on its own
+// tick alone, so it is formed once, when the tick's slice is done (k_rp_tick), and kept
+// in a ring; the slices themselves are not kept.  The correction is a GEMM per block,
+// (N x bn*tw) X times (bn*tw x bn) K on v_mfma_f32_32x32x2f32 (k_rp_corr), its reduction
+// split over workgroups where the output alone does not fill the chip; k_rp_finish then
+// adds the splits.  A tick is two or three launches: k_rp_corr (with the previous tick's
+// dx on blocks of its own), k_rp_finish (splits, or no correction), k_rp_tick (clip
+// decision, w_tick, dw, X).  The base term is made for kBaseTicks ticks at a time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -55,309 +57,384 @@ __global__ void k_lr_capture(CaptureArgs C, int sample, int lr) {
 }
 
 // ---------------------------------------------------------------- base term
-// replay_base_blocks_kernel (replay_dw_dx.cu:227-274): one thread per (i, j)
-// of a diagonal block, taps summed in time order with fused multiply-adds.
-__global__ void k_rp_base(ReplayBaseArgs A) {
+// replay_base_blocks_kernel (replay_dw_dx.cu:227-274): one thread per (i, j) of a
+// diagonal block and kBaseTicks ticks, taps summed in time order with fused multiply-adds.
+// The taps (64 MB for 16 blocks of 128 and K_len 64) are read once for all those ticks:
+// 16 us a tick when made tick by tick, 2.6 us now.
+__global__ void __launch_bounds__(kThreads) k_rp_base(ReplayBaseArgs A) {
     const int b = blockIdx.y;
-    const int bn = A.bn[b];
+    const int bn = A.bn[b], bnp = A.bnp[b];
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b == 0 && e == 0) A.slot_scale[A.cur] = 1.f;
     if (e >= bn * bn) return;
     const int bi = e / bn;
     const int row = A.start[b] + bi;
-    const float* K = A.kt1 + A.koff[b];
-    const size_t plane = static_cast<size_t>(bn) * bn;
-    float sum = 0.f;
-    for (int u = 0; u < A.tw; ++u)
-        sum = fmaf(K[static_cast<size_t>(A.k_t0 + u) * plane + e],
-                   A.it[static_cast<size_t>(A.it_t0 + u) * A.N + row], sum);
-    A.base[A.boff[b] + e] = sum * A.dt * (*A.gs);
+    const float* K = A.kp + A.koff[b] + static_cast<size_t>(bi) * bnp + (e - bi * bn);
+    const size_t plane = static_cast<size_t>(bn) * bnp;
+    float sum[kBaseTicks];
+#pragma unroll
+    for (int g = 0; g < kBaseTicks; ++g) sum[g] = 0.f;
+    // tap k0 + p of tick t0 + g meets the signal at time tau0 + p + g: a group of kBaseTicks
+    // taps needs 2 kBaseTicks - 1 signals, of which the last group brought the first half.
+    // Times before the first signal (and taps past the last) are skipped, so whatever is
+    // loaded in their place is not used.
+    const int first = A.t0 + A.ng - 1 < A.K_len ? A.K_len - (A.t0 + A.ng - 1) : 0;
+    auto signal = [&](int tau) { return A.it[static_cast<size_t>(min(max(tau, 0), A.T - 1)) * A.N + row]; };
+    float w[2 * kBaseTicks];
+#pragma unroll
+    for (int g = 0; g < kBaseTicks; ++g) w[kBaseTicks + g] = signal(A.t0 + first - A.K_len + 1 + g);
+    for (int k0 = first; k0 < A.K_len; k0 += kBaseTicks) {
+        const int tau0 = A.t0 + k0 - A.K_len + 1;
+        float k[kBaseTicks];
+#pragma unroll
+        for (int p = 0; p < kBaseTicks; ++p) {
+            k[p] = K[min(k0 + p, A.K_len - 1) * plane];
+            w[p] = w[kBaseTicks + p];
+            w[kBaseTicks + p] = signal(tau0 + kBaseTicks + p);
+        }
+#pragma unroll
+        for (int p = 0; p < kBaseTicks; ++p)
+#pragma unroll
+            for (int g = 0; g < kBaseTicks; ++g)
+                if (k0 + p < A.K_len && tau0 + p + g >= 1) sum[g] = fmaf(k[p], w[p + g], sum[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < kBaseTicks; ++g)
+        if (g < A.ng) A.base[g * A.base_stride + A.boff[b] + e] = sum[g];
+}
+
+// Fixed-order sum over the workgroup (kT threads) of x; every thread gets it.
+template <int kT, class V>
+__device__ __forceinline__ V block_sum(V x, V* sh) {
+    const int tid = threadIdx.x;
+    sh[tid] = x;
+    __syncthreads();
+#pragma unroll
+    for (int st = kT / 2; st > 0; st >>= 1) {
+        if (tid < st) sh[tid] += sh[tid + st];
+        __syncthreads();
+    }
+    const V r = sh[0];
+    __syncthreads();
+    return r;
+}
+
+// One element of a tick's slice from its correction sum c (replay_dw_dx.cu:227-325): base
+// term added inside the row's own block; on clip ticks non-finite entries become 0 and the
+// square goes to the norm.
+__device__ __forceinline__ float rp_element(const ReplayOut& O, float c, int row, int col, int s, int bn,
+                                            const float* base, float gs, double& sq) {
+    float v = c * O.dt;
+    if (row >= s && row < s + bn) v = base[static_cast<size_t>(row - s) * bn + col - s] * O.dt * gs + v;
+    if (O.sanitize) {
+        if (!isfinite(v)) v = 0.f;
+        sq += static_cast<double>(v) * v;
+    }
+    return v;
+}
+
+// ---------------------------------------------------------------- dx
+// replay_dx_reduce_kernel / replay_dx_finalize_kernel (replay_dw_dx.cu:445-501): one
+// workgroup per input column, fixed-order reduction.  A clip at that tick also rescales
+// the input's earlier dx entries (LearnRuntime.cpp:2257).  A tick's dx needs the whole
+// w_tick, so it rides on the next tick's first launch (a launch of its own: 3.2-5.3 us).
+template <int kT>
+__device__ __forceinline__ void rp_dx(const ReplayDx& X, int N, int j, float* sh) {
+    const int tid = threadIdx.x;
+    const int p = X.pin[j];
+    const float sig = X.clip_ran ? *X.tick_scale : 1.f;
+    float s = 0.f, bsum = 0.f;
+    for (int i = tid; i < N; i += kT) {
+        const float v = X.cur[static_cast<size_t>(i) * N + p] * sig;
+        bsum += v;
+        s += X.w_tick[i] / (v + X.eps);
+    }
+    const float st = block_sum<kT>(s, sh);
+    const float bt = block_sum<kT>(bsum, sh);
+    float* row = X.dx + static_cast<size_t>(j) * X.ksteps;
+    if (X.clip_ran && sig != 1.f)
+        for (int t = tid; t < X.t_idx; t += kT) row[t] *= sig;
+    if (tid == 0) row[X.t_idx] = st * bt;
+}
+
+__global__ void __launch_bounds__(kThreads) k_rp_dx(ReplayDx X, int N) {
+    __shared__ float sh[kThreads];
+    rp_dx<kThreads>(X, N, blockIdx.x, sh);
 }
 
 // ---------------------------------------------------------------- correction GEMM
-// Workgroup tile: 128 rows x TJ columns of one block (TJ = 64 or 128) with NT
-// threads, the waves arranged as WR row groups x (NT/64/WR) column groups; a
-// wave owns a (128/WR) x (TJ/WC) sub-tile, held as 32 x 32 accumulators of
-// v_mfma_f32_32x32x2f32.  The reduction runs over (tap u, chunk of KC columns
-// k).  Each chunk stages X -- formed from the history slice D and its
-// column-gathered copy G, both read as contiguous row segments -- and the K
-// taps through LDS, double-buffered, with the next chunk's global loads in
-// flight while the MFMAs run.
-// Measured on MI355X (N = 2048, 16 blocks of 128, K_len 64): 64-tap chunks
-// (one 130 KB workgroup per CU) beat 32- and 16-tap chunks, and 8 waves of
-// 32 x 64 sub-tiles beat 4 waves of 64 x 64.
-constexpr int kCorrThreads = 512;
+// Workgroup tile: kTI rows x TJ columns of one block over a range of the reduction,
+// kT threads, one 32 x (TJ/WC) sub-tile per wave.  The reduction index runs over (tap u,
+// column k of the block padded to a multiple of 4), flattened, in chunks of kKC, so narrow
+// blocks fill a chunk with several taps.  A chunk's X rows and taps are read as 16-byte
+// groups (X ring and taps are both k-contiguous and padded with zeros, so nothing needs a
+// mask but the end of the range), held in registers while the previous chunk's MFMAs run
+// and staged through LDS, double-buffered; rows are kKC + 4 floats apart, which spreads a
+// wave's ds_read_b128 over all banks.  Each such read feeds four MFMAs: which of the four
+// k a step takes is the same for both operands.
+// Bound: the fp32 matrix cores (157 TFLOP/s; a library product of 8192^3 reaches 153).
+// N = 2048 in 16 blocks of 128, K_len 64: 630 -> 439 us a launch over 128 ticks, 118
+// TFLOP/s with the window full (before: X formed while staging from two history rings, one
+// element per load).  Chunks of 32 with two workgroups per CU: 3% slower.
 constexpr int kTI = 128;
 constexpr int kKC = 64;
-constexpr int kWR = 4;
-constexpr int kAPad = kTI + 1;
+constexpr int kLd = kKC + 4;
 
 template <int TJ>
-__global__ __launch_bounds__(kCorrThreads) void k_rp_corr(ReplayCorrArgs A) {
-    constexpr int NW = kCorrThreads / 64;               // waves
-    constexpr int WC = NW / kWR;                        // column groups of waves
-    constexpr int WTI = kTI / kWR, WTJ = TJ / WC;       // wave sub-tile
-    constexpr int MR = WTI / 32, NC = WTJ / 32;         // accumulators per wave
-    static_assert(MR >= 1 && NC >= 1 && WTI % 32 == 0 && WTJ % 32 == 0, "wave sub-tile must be 32-aligned");
-    constexpr int ASTEP = kCorrThreads / kKC;           // A rows covered per pass
-    constexpr int RA = kTI / ASTEP;                     // A elements per thread and array
-    constexpr int BSTEP = kCorrThreads / TJ;            // B taps covered per pass
-    constexpr int BR = kKC / BSTEP;                     // B elements per thread
-    __shared__ float As[2][kKC][kAPad];                 // X chunk, [k][i]
-    __shared__ float Bs[2][kKC][TJ];                    // K chunk, [k][j]
-    __shared__ double red_s[NW];
-    __shared__ int red_f[NW];
+struct CorrShape {
+    static constexpr int kT = TJ == 32 ? 256 : 512;     // threads
+    static constexpr int NW = kT / 64;
+    static constexpr int WC = TJ == 32 ? 1 : 2;         // column groups of waves
+    static constexpr int WR = NW / WC;                  // row groups: 32 rows each
+    static constexpr int NC = TJ / WC / 32;             // accumulators per wave
+    static constexpr int RS = kT / (kKC / 4);           // rows apart that a thread stages
+    static constexpr int GA = kTI * kKC / 4 / kT;       // 16-byte groups of X per thread and chunk
+    static constexpr int GB = TJ * kKC / 4 / kT;        // and of taps
+    static_assert(WR * 32 == kTI && NC >= 1 && GA >= 1 && GB >= 1, "tile does not divide over the waves");
+};
 
-    const int2 tl = A.tiles[blockIdx.x];
-    const int b = tl.x, j0 = tl.y;
-    const int s = A.start[b], bn = A.bn[b];
-    const int N = A.N;
-    const int i0 = blockIdx.y * kTI;
+// kPart: write the sums of this split to the partials; otherwise the tick's slice itself.
+template <int TJ, bool kPart>
+__global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A) {
+    using S = CorrShape<TJ>;
+    __shared__ __align__(16) float As[2][kTI][kLd];
+    __shared__ __align__(16) float Bs[2][TJ][kLd];
+    __shared__ double red_s[S::NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave / WC, wc = wave % WC;
-    const float* Kb = A.kt2 + A.koff[b];
-    const size_t plane = static_cast<size_t>(bn) * bn;
-    const int nkc = (bn + kKC - 1) / kKC;
-    const int nchunk = A.tw * nkc;
+    if (static_cast<int>(blockIdx.x) >= A.ncorr) {            // the previous tick's dx
+        rp_dx<S::kT>(A.dx, A.O.N, blockIdx.x - A.ncorr, &As[0][0][0]);
+        return;
+    }
+    // workgroups go to the eight XCDs in turn: give each XCD a run of consecutive tiles, so
+    // the row tiles that share a block's taps read them from one L2
+    int wg = blockIdx.x;
+    if (A.ncorr % 8 == 0) wg = (wg & 7) * (A.ncorr >> 3) + (wg >> 3);
+    const int rt = wg % A.row_tiles;
+    const int q = wg / A.row_tiles;
+    const int sp = q % A.nsplit;
+    const int2 tl = A.tiles[q / A.nsplit];
+    const int b = tl.x, j0 = tl.y;
+    const int s = A.start[b], bn = A.bn[b], bnp = A.bnp[b];
+    const int N = A.O.N;
+    const int i0 = rt * kTI;
+    const int nb4 = bnp >> 2;
+    const int total = A.tw * nb4;                             // 16-byte groups of the reduction
+    const int nchunk = (total + kKC / 4 - 1) / (kKC / 4);
+    const int c0 = static_cast<int>(static_cast<long long>(nchunk) * sp / A.nsplit);
+    const int c1 = static_cast<int>(static_cast<long long>(nchunk) * (sp + 1) / A.nsplit);
 
-    // staging coordinates: A element (row ai + ASTEP r, tap ak), B element (tap bk + BSTEP r, column bj)
-    const int ak = tid % kKC, ai = tid / kKC;
-    const int bj = tid % TJ, bk = tid / TJ;
-    float rd[RA], rg[RA], rb[BR];
-    float ca = 0.f, cp = 0.f;
-
+    const int kg = tid % (kKC / 4), r0 = tid / (kKC / 4);     // group within the chunk, first row
+    const float* Xb = A.x + static_cast<long long>(A.xoff[b]);
+    const float* Kb = A.kp + A.koff[b];
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4 ra[S::GA], rb[S::GB];
+    float sig = 0.f;
+    bool in = false;
+    // only loads here: the first use of what they bring is in stage(), behind the MFMAs
     auto fetch = [&](int c) {
-        const int u = c / nkc;
-        const int k0 = (c - u * nkc) * kKC;
-        const int h = (A.t_lr - A.tw + u) % A.R;
-        const size_t hoff = static_cast<size_t>(h) * A.slice;
-        const float* D = A.hist + hoff;
-        const float* G = A.ghist + hoff;
-        const int kc = k0 + ak;
-        const bool kin = kc < bn;
-        const int col = s + kc;
-        const size_t tau = static_cast<size_t>(A.it_t0 + u);
-        ca = 0.f;
-        cp = 0.f;
-        if (kin) {
-            const float sig = A.slot_scale[h];
-            ca = sig * A.dv[tau * N + col];
-            cp = sig * A.dp[tau * N + col];
+        const int pos = c * (kKC / 4) + kg;
+        const int u = pos / nb4;
+        const int k = (pos - u * nb4) * 4;
+        in = pos < total;
+        int h = A.h0 + (in ? u : 0);
+        if (h >= A.R) h -= A.R;
+        sig = A.slot_scale[h];
+        const float* X = Xb + h * A.xslice + (in ? k : 0);
+        const float* K = Kb + static_cast<size_t>(A.k_t0 + (in ? u : 0)) * bn * bnp + (in ? k : 0);
+#pragma unroll
+        for (int r = 0; r < S::GA; ++r) {
+            const int i = min(i0 + r0 + S::RS * r, N - 1);
+            // the history streams through once per tick: keep it out of the caches, so that
+            // the taps, reused by every row tile, stay in L2
+            ra[r] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(X + static_cast<size_t>(i) * bnp));
         }
 #pragma unroll
-        for (int r = 0; r < RA; ++r) {
-            const int i = i0 + ai + ASTEP * r;
-            float x = 0.f, y = 0.f;
-            if (kin && i < N) {
-                const size_t o = static_cast<size_t>(i) * N + col;
-                // the history window streams through once per tick: keep it out of
-                // the caches so the K taps, reused by every row tile, stay in L2
-                x = __builtin_nontemporal_load(D + o);
-                y = __builtin_nontemporal_load(G + o);
-            }
-            rd[r] = x;
-            rg[r] = y;
-        }
-        const float* Kt = Kb + static_cast<size_t>(A.k_t0 + u) * plane;
-        const int jj = j0 + bj;
-#pragma unroll
-        for (int r = 0; r < BR; ++r) {
-            const int k = k0 + bk + BSTEP * r;
-            rb[r] = (jj < bn && k < bn) ? Kt[static_cast<size_t>(k) * bn + jj] : 0.f;
+        for (int r = 0; r < S::GB; ++r) {
+            const int j = min(j0 + r0 + S::RS * r, bn - 1);
+            rb[r] = *reinterpret_cast<const f4*>(K + static_cast<size_t>(j) * bnp);
         }
     };
     auto stage = [&](int buf) {
+        const f4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < RA; ++r) As[buf][ak][ai + ASTEP * r] = rd[r] * ca + rg[r] * cp;
+        for (int r = 0; r < S::GA; ++r)
+            *reinterpret_cast<f4*>(&As[buf][r0 + S::RS * r][kg * 4]) = in ? ra[r] * sig : zero;
 #pragma unroll
-        for (int r = 0; r < BR; ++r) Bs[buf][bk + BSTEP * r][bj] = rb[r];
+        for (int r = 0; r < S::GB; ++r)
+            *reinterpret_cast<f4*>(&Bs[buf][r0 + S::RS * r][kg * 4]) = in ? rb[r] : zero;
     };
 
-    f16v acc[MR][NC];
+    const int wr = wave / S::WC, wc = wave % S::WC;
+    f16v acc[S::NC];
 #pragma unroll
-    for (int m = 0; m < MR; ++m)
+    for (int n = 0; n < S::NC; ++n)
 #pragma unroll
-        for (int n = 0; n < NC; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
-
-    if (nchunk > 0) {
-        fetch(0);
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+    if (c1 > c0) {
+        fetch(c0);
         stage(0);
         __syncthreads();
-        const int kr = lane >> 5;
-        const int ia = wr * WTI + (lane & 31);
-        const int jb = wc * WTJ + (lane & 31);
-        for (int c = 0; c < nchunk; ++c) {
-            const int buf = c & 1;
-            if (c + 1 < nchunk) fetch(c + 1);
+        const int kr = (lane >> 5) * 4;
+        const int ia = wr * 32 + (lane & 31);
+        const int jb = wc * 32 * S::NC + (lane & 31);
+        for (int c = c0; c < c1; ++c) {
+            const int buf = (c - c0) & 1;
+            if (c + 1 < c1) fetch(c + 1);
 #pragma unroll
-            for (int q = 0; q < kKC / 2; ++q) {
-                float av[MR], bv[NC];
+            for (int g = 0; g < kKC / 8; ++g) {
+                const float4 av = *reinterpret_cast<const float4*>(&As[buf][ia][8 * g + kr]);
+                float4 bv[S::NC];
 #pragma unroll
-                for (int m = 0; m < MR; ++m) av[m] = As[buf][2 * q + kr][ia + 32 * m];
+                for (int n = 0; n < S::NC; ++n)
+                    bv[n] = *reinterpret_cast<const float4*>(&Bs[buf][jb + 32 * n][8 * g + kr]);
+                const float a4[4] = {av.x, av.y, av.z, av.w};
 #pragma unroll
-                for (int n = 0; n < NC; ++n) bv[n] = Bs[buf][2 * q + kr][jb + 32 * n];
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int m = 0; m < MR; ++m)
-#pragma unroll
-                    for (int n = 0; n < NC; ++n)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[m], bv[n], acc[m][n], 0, 0, 0);
+                    for (int n = 0; n < S::NC; ++n) {
+                        const float b4[4] = {bv[n].x, bv[n].y, bv[n].z, bv[n].w};
+                        acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[e], b4[e], acc[n], 0, 0, 0);
+                    }
             }
-            if (c + 1 < nchunk) stage(buf ^ 1);
+            if (c + 1 < c1) stage(buf ^ 1);
             __syncthreads();
         }
     }
 
-    // epilogue: accumulator (m, n) of a lane holds rows 32m + 8(r/4) + 4(lane/32) + r%4
-    // and column 32n + lane%32 of its wave's sub-tile
+    // accumulator n of a lane holds rows 8(r/4) + 4(lane/32) + r%4 and column 32n + lane%32
+    // of its wave's sub-tile
     double sq = 0.0;
-    int bad = 0;
-    const float* base = A.base + A.boff[b];
+    const float gs = *A.O.gs;
+    const float* base = A.O.base + A.boff[b];
+    float* out = kPart ? A.part + static_cast<size_t>(sp) * N * N : A.O.out;
 #pragma unroll
-    for (int m = 0; m < MR; ++m)
+    for (int n = 0; n < S::NC; ++n) {
+        const int jw = j0 + (wc * S::NC + n) * 32 + (lane & 31);
 #pragma unroll
-        for (int n = 0; n < NC; ++n) {
-            const int jw = j0 + wc * WTJ + 32 * n + (lane & 31);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = i0 + wr * WTI + 32 * m + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row >= N || jw >= bn) continue;
-                float v = acc[m][n][r] * A.dt;
-                if (row >= s && row < s + bn) v = base[static_cast<size_t>(row - s) * bn + jw] + v;
-                if (A.sanitize) {
-                    if (!isfinite(v)) {
-                        v = 0.f;
-                        bad = 1;
-                    }
-                    sq += static_cast<double>(v) * v;
-                }
-                A.out[static_cast<size_t>(row) * N + s + jw] = v;
-            }
+        for (int r = 0; r < 16; ++r) {
+            const int row = i0 + wr * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (row >= N || jw >= bn) continue;
+            out[static_cast<size_t>(row) * N + s + jw] =
+                kPart ? acc[n][r] : rp_element(A.O, acc[n][r], row, s + jw, s, bn, base, gs, sq);
         }
-    if (A.sanitize) {
-        for (int o = 32; o > 0; o >>= 1) {
-            sq += __shfl_xor(sq, o);
-            bad |= __shfl_xor(bad, o);
-        }
-        if (lane == 0) {
-            red_s[wave] = sq;
-            red_f[wave] = bad;
-        }
+    }
+    if (!kPart && A.O.sanitize) {
+        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+        if (lane == 0) red_s[wave] = sq;
         __syncthreads();
         if (tid == 0) {
             double t = 0.0;
-            int f = 0;
-            for (int w = 0; w < NW; ++w) {
-                t += red_s[w];
-                f |= red_f[w];
-            }
-            const int wg = blockIdx.y * gridDim.x + blockIdx.x;
-            A.norm_part[wg] = t;
-            A.flag_part[wg] = f;
+            for (int w = 0; w < S::NW; ++w) t += red_s[w];
+            A.O.norm_part[wg] = t;
         }
     }
 }
 
-// G[i][c] = D[i][pre(c)] (0 without a pre column): the column-gathered copy of
-// a new history slice, so the correction reads both operands row-contiguous.
-__global__ void k_rp_pregather(const float* D, const int* pre, int N, float* G) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= N) return;
-    const size_t row = static_cast<size_t>(blockIdx.y) * N;
-    const int p = pre[c];
-    G[row + c] = p >= 0 ? D[row + p] : 0.f;
-}
-
-// ---------------------------------------------------------------- clip
-// replay_frobenius_*_kernel (replay_dw_dx.cu:28-93) and the driver's decision
-// (LearnRuntime.cpp:2238-2262): l2 over the finite entries; above the
-// threshold the tick's slice, the history, the accumulators and the grad
-// scale are all multiplied by thr / l2.  The decision stays on the device.
-__global__ void k_rp_clip(const double* part, const int* flag, int n, float thr, float* gs, float* slot_scale,
-                          int R, float* tick_scale) {
+// The tick's slice from the correction's split sums, added in split order (nsplit 0: no
+// correction), kE elements per thread; the previous tick's dx on blocks of its own.  The
+// splits are read four at a time, so a thread has 4 kE loads in flight (one at a time,
+// waiting for each, the kernel took 52 us at N = 400 with 28 splits).
+template <int kE>
+__global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
     __shared__ double sh[kThreads];
-    __shared__ float sc_sh;
-    const int tid = threadIdx.x;
-    double acc = 0.0;
-    for (int q = tid; q < n; q += kThreads) acc += part[q];
-    sh[tid] = acc;
-    __syncthreads();
-    for (int st = kThreads / 2; st > 0; st >>= 1) {
-        if (tid < st) sh[tid] += sh[tid + st];
-        __syncthreads();
+    if (static_cast<int>(blockIdx.x) >= A.nblock) {
+        rp_dx<kThreads>(A.dx, A.O.N, blockIdx.x - A.nblock, reinterpret_cast<float*>(sh));
+        return;
     }
-    if (tid == 0) {
-        const double l2 = sqrt(fmax(0.0, sh[0]));
-        float sc = 1.f;
-        if (l2 > static_cast<double>(thr) && isfinite(l2)) sc = static_cast<float>(static_cast<double>(thr) / l2);
-        *tick_scale = sc;
-        if (sc != 1.f) *gs *= sc;
-        sc_sh = sc;
+    const unsigned N = A.O.N, total = N * N;
+    const unsigned e0 = blockIdx.x * kE * kThreads + threadIdx.x;
+    const float gs = *A.O.gs;
+    float c[kE];
+    unsigned at[kE];
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+        c[r] = 0.f;
+        at[r] = min(e0 + r * kThreads, total - 1);
     }
-    __syncthreads();
-    const float sc = sc_sh;
-    if (sc != 1.f)
-        for (int r = tid; r < R; r += kThreads) slot_scale[r] *= sc;
-    (void)flag;
+    int sp = 0;
+    for (; sp + 4 <= A.nsplit; sp += 4) {
+        float x[4][kE];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < kE; ++r) x[q][r] = A.part[static_cast<size_t>(sp + q) * total + at[r]];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < kE; ++r) c[r] += x[q][r];
+    }
+    for (; sp < A.nsplit; ++sp)
+#pragma unroll
+        for (int r = 0; r < kE; ++r) c[r] += A.part[static_cast<size_t>(sp) * total + at[r]];
+    double sq = 0.0;
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+        if (e0 + r * kThreads >= total) break;
+        const unsigned row = at[r] / N, col = at[r] - row * N;
+        const int b = A.col_block[col];
+        A.O.out[at[r]] = rp_element(A.O, c[r], row, col, A.start[b], A.bn[b], A.O.base + A.boff[b], gs, sq);
+    }
+    if (A.O.sanitize) {
+        const double t = block_sum<kThreads>(sq, sh);
+        if (threadIdx.x == 0) A.O.norm_part[blockIdx.x] = t;
+    }
 }
 
-// ---------------------------------------------------------------- w_tick
-// replay_compute_w_tick_kernel (replay_dw_dx.cu:96-114): one wave per row.
-__global__ void k_rp_wtick(const float* cur, const float* slot_scale, int cur_slot, int N, const int* po,
-                           int n_out, const float* dl, int clip_ran, const float* tick_scale, float* w_tick,
-                           float* dw_acc) {
-    const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+// ---------------------------------------------------------------- a tick's end
+// The Frobenius clip (replay_frobenius_*_kernel replay_dw_dx.cu:28-93, the driver's
+// decision LearnRuntime.cpp:2238-2262): l2 over the finite entries; above the threshold
+// the tick's slice, the history, the accumulators and the grad scale are all multiplied
+// by thr / l2.  Every workgroup that needs the factor sums the norm's partials itself, in
+// the same order (a launch of its own took 4 us); block 0 stores it with the rescaled
+// scales, which only later launches read.  w_tick (replay_dw_dx.cu:96-114): one wave per
+// row.  The remaining blocks form X of this tick from its slice.
+constexpr int kGather = 4;
+__global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
+    __shared__ double sh[kThreads];
+    const int tid = threadIdx.x;
+    const unsigned N = A.N;
+    if (static_cast<int>(blockIdx.x) >= A.wblocks) {
+        const unsigned total = N * N;
+        const unsigned e0 = (blockIdx.x - A.wblocks) * kGather * kThreads + tid;
+#pragma unroll
+        for (int r = 0; r < kGather; ++r) {
+            const unsigned e = e0 + r * kThreads;
+            if (e >= total) break;
+            const unsigned row = e / N, c = e - row * N;
+            const int p = A.pre[c], b = A.col_block[c];
+            const float g = p >= 0 ? A.cur[static_cast<size_t>(row) * N + p] : 0.f;
+            A.x[A.xoff[b] + static_cast<size_t>(row) * A.bnp[b] + c - A.start[b]] =
+                A.cur[e] * A.dv[c] + g * A.dp[c];
+        }
+        return;
+    }
+    float sc = 1.f;
+    if (A.due) {
+        double acc = 0.0;
+        for (int q = tid; q < A.npart; q += kThreads) acc += A.norm_part[q];
+        const double l2 = sqrt(fmax(0.0, block_sum<kThreads>(acc, sh)));
+        if (l2 > static_cast<double>(A.thr) && isfinite(l2)) sc = static_cast<float>(static_cast<double>(A.thr) / l2);
+    }
+    if (blockIdx.x == 0) {
+        if (A.due && tid == 0) {
+            *A.tick_scale = sc;
+            if (sc != 1.f) *A.gs *= sc;
+        }
+        for (int r = tid; r < A.R; r += kThreads) {
+            if (r == A.cur_slot) A.slot_scale[r] = sc;
+            else if (sc != 1.f) A.slot_scale[r] *= sc;
+        }
+    }
+    const unsigned row = blockIdx.x * (kThreads / 64) + (tid >> 6);
+    const int lane = tid & 63;
     if (row >= N) return;
-    const float sig = slot_scale[cur_slot];
-    const float* r = cur + static_cast<size_t>(row) * N;
+    const float* r = A.cur + static_cast<size_t>(row) * N;
     float acc = 0.f;
-    for (int o = lane; o < n_out; o += 64) acc = fmaf(r[po[o]] * sig, dl[o], acc);
+    for (int o = lane; o < A.n_out; o += 64) acc = fmaf(r[A.po[o]] * sc, A.dl[o], acc);
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
     if (lane == 0) {
-        const float ts = clip_ran ? *tick_scale : 1.f;
-        w_tick[row] = acc;
-        dw_acc[row] = dw_acc[row] * ts + acc;
+        A.w_tick[row] = acc;
+        A.dw_acc[row] = A.dw_acc[row] * sc + acc;
     }
-}
-
-// ---------------------------------------------------------------- dx
-// replay_dx_reduce_kernel / replay_dx_finalize_kernel (replay_dw_dx.cu:445-501):
-// one workgroup per input column, fixed-order reduction.  A clip at this tick
-// also rescales the input's earlier dx entries (LearnRuntime.cpp:2257).
-__global__ void k_rp_dx(const float* cur, const float* slot_scale, int cur_slot, int N, const int* pin, int n_in,
-                        const float* w_tick, float eps, int t_idx, int ksteps, int clip_ran, const float* tick_scale,
-                        float* dx) {
-    __shared__ float s_sh[kThreads], b_sh[kThreads];
-    const int j = blockIdx.x;
-    const int tid = threadIdx.x;
-    if (j >= n_in) return;
-    const int p = pin[j];
-    const float sig = slot_scale[cur_slot];
-    float s = 0.f, bsum = 0.f;
-    for (int i = tid; i < N; i += kThreads) {
-        const float v = cur[static_cast<size_t>(i) * N + p] * sig;
-        bsum += v;
-        s += w_tick[i] / (v + eps);
-    }
-    s_sh[tid] = s;
-    b_sh[tid] = bsum;
-    __syncthreads();
-    for (int st = kThreads / 2; st > 0; st >>= 1) {
-        if (tid < st) {
-            s_sh[tid] += s_sh[tid + st];
-            b_sh[tid] += b_sh[tid + st];
-        }
-        __syncthreads();
-    }
-    float* row = dx + static_cast<size_t>(j) * ksteps;
-    if (clip_ran) {
-        const float ts = *tick_scale;
-        if (ts != 1.f)
-            for (int t = tid; t < t_idx; t += kThreads) row[t] *= ts;
-    }
-    if (tid == 0) row[t_idx] = s_sh[0] * b_sh[0];
 }
 
 __global__ void k_rp_scale_into(const float* src, float scale, float* dst, long long n) {
@@ -400,37 +477,63 @@ void launch_rp_base(const ReplayBaseArgs& a, int nblk, int max_bn, hipStream_t s
 
 int rp_corr_row_tiles(int N) { return (N + kTI - 1) / kTI; }
 
-void launch_rp_corr(const ReplayCorrArgs& a, int ntiles, int tile_cols, hipStream_t s) {
-    const dim3 grid(ntiles, rp_corr_row_tiles(a.N));
-    if (tile_cols == 128)
-        hipLaunchKernelGGL(k_rp_corr<128>, grid, dim3(kCorrThreads), 0, s, a);
-    else
-        hipLaunchKernelGGL(k_rp_corr<64>, grid, dim3(kCorrThreads), 0, s, a);
+// Workgroups the reduction is split over: enough for one on every CU, as long as each
+// keeps a chunk.  Problem sizes alone decide, so every entry point sums in the same order.
+// N = 96, K_len 8: 34 -> 6 us a launch (2 tiles, one workgroup each before); N = 701,
+// K_len 24: 307 -> 32 us (36 tiles); N = 2048 has a tile per CU and is not split.
+int rp_corr_splits(int N, int ntiles, int max_bnp, int tw) {
+    const int wgs = ntiles * rp_corr_row_tiles(N);
+    const long long chunks = (static_cast<long long>(tw) * max_bnp + kKC - 1) / kKC;
+    const long long want = std::min<long long>(256 / std::max(wgs, 1), chunks);
+    return static_cast<int>(std::max<long long>(want, 1));
 }
 
-void launch_rp_pregather(const float* D, const int* pre, int N, float* G, hipStream_t s) {
-    hipLaunchKernelGGL(k_rp_pregather, dim3((N + kThreads - 1) / kThreads, N), dim3(kThreads), 0, s, D, pre, N, G);
+template <int TJ>
+void launch_corr_tile(const ReplayCorrArgs& a, hipStream_t s) {
+    const dim3 grid(a.ncorr + a.dx.n_in), block(CorrShape<TJ>::kT);
+    if (a.nsplit > 1) hipLaunchKernelGGL((k_rp_corr<TJ, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_rp_corr<TJ, false>), grid, block, 0, s, a);
 }
 
-void launch_rp_clip(const double* part, const int* flag, int n, float thr, float* gs, float* slot_scale, int R,
-                    float* tick_scale, hipStream_t s) {
-    hipLaunchKernelGGL(k_rp_clip, dim3(1), dim3(kThreads), 0, s, part, flag, n, thr, gs, slot_scale, R, tick_scale);
+void launch_rp_corr(const ReplayCorrArgs& a, int tile_cols, hipStream_t s) {
+    if (tile_cols == 128) launch_corr_tile<128>(a, s);
+    else if (tile_cols == 64) launch_corr_tile<64>(a, s);
+    else launch_corr_tile<32>(a, s);
 }
 
-void launch_rp_wtick(const float* cur, const float* slot_scale, int cur_slot, int N, const int* po, int n_out,
-                     const float* dl, int clip_ran, const float* tick_scale, float* w_tick, float* dw_acc,
-                     hipStream_t s) {
-    const int rows_per = kThreads / 64;
-    hipLaunchKernelGGL(k_rp_wtick, dim3((N + rows_per - 1) / rows_per), dim3(kThreads), 0, s, cur, slot_scale,
-                       cur_slot, N, po, n_out, dl, clip_ran, tick_scale, w_tick, dw_acc);
+// Elements per thread of k_rp_finish: one while that gives no more than about 1024 blocks
+// (every w_tick workgroup adds up the blocks' norm partials), then as many as keep it so.
+static int finish_elems(int N) {
+    const long long blocks = (static_cast<long long>(N) * N + kThreads - 1) / kThreads;
+    return blocks <= 1024 ? 1 : blocks <= 4096 ? 4 : blocks <= 16384 ? 8 : 16;
 }
 
-void launch_rp_dx(const float* cur, const float* slot_scale, int cur_slot, int N, const int* pin, int n_in,
-                  const float* w_tick, float eps, int t_idx, int ksteps, int clip_ran, const float* tick_scale,
-                  float* dx, hipStream_t s) {
-    if (n_in <= 0) return;
-    hipLaunchKernelGGL(k_rp_dx, dim3(n_in), dim3(kThreads), 0, s, cur, slot_scale, cur_slot, N, pin, n_in, w_tick,
-                       eps, t_idx, ksteps, clip_ran, tick_scale, dx);
+int rp_finish_blocks(int N) {
+    const long long per = static_cast<long long>(finish_elems(N)) * kThreads;
+    return static_cast<int>((static_cast<long long>(N) * N + per - 1) / per);
+}
+
+void launch_rp_finish(ReplayFinishArgs a, hipStream_t s) {
+    a.nblock = rp_finish_blocks(a.O.N);
+    const dim3 grid(a.nblock + a.dx.n_in);
+    switch (finish_elems(a.O.N)) {
+        case 1: hipLaunchKernelGGL(k_rp_finish<1>, grid, dim3(kThreads), 0, s, a); break;
+        case 4: hipLaunchKernelGGL(k_rp_finish<4>, grid, dim3(kThreads), 0, s, a); break;
+        case 8: hipLaunchKernelGGL(k_rp_finish<8>, grid, dim3(kThreads), 0, s, a); break;
+        default: hipLaunchKernelGGL(k_rp_finish<16>, grid, dim3(kThreads), 0, s, a); break;
+    }
+}
+
+void launch_rp_tick(ReplayTickArgs a, hipStream_t s) {
+    const long long per = static_cast<long long>(kGather) * kThreads;
+    a.wblocks = a.dl ? (a.N + kThreads / 64 - 1) / (kThreads / 64) : 0;
+    const long long gather = a.x ? (static_cast<long long>(a.N) * a.N + per - 1) / per : 0;
+    if (a.wblocks + gather > 0)
+        hipLaunchKernelGGL(k_rp_tick, dim3(static_cast<unsigned>(a.wblocks + gather)), dim3(kThreads), 0, s, a);
+}
+
+void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s) {
+    if (a.n_in > 0) hipLaunchKernelGGL(k_rp_dx, dim3(a.n_in), dim3(kThreads), 0, s, a, N);
 }
 
 void launch_rp_scale_into(const float* src, float scale, float* dst, long long n, hipStream_t s) {

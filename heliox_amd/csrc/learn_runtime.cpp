@@ -1,8 +1,8 @@
 // Host side of the learn gradient surface: dense blocks, the capture session
 // and the per-tick LRDS replay driver (LearnRuntime.cpp:197-257, 1619-2457).
 //
-// The replay loop issues, per LR tick, base -> correction GEMM -> [clip] ->
-// w_tick -> [dx] on one stream with no host synchronisation: the Frobenius
+// The replay loop issues, per LR tick, correction GEMM [-> its splits' sum] -> tick end
+// (clip decision, w_tick, X) on one stream with no host synchronisation: the Frobenius
 // clip decision, the grad scale and the history rescale stay on the device
 // (the reference copies the norm to the host every checked tick).
 #include <hip/hip_runtime.h>
@@ -80,15 +80,19 @@ void LearnRuntime::clear_dense_blocks() {
     free_all(ws_mem_);
     free_all(sig_mem_);
     ws_key_.clear();
-    k_len_ = nblk_ = max_bn_ = 0;
+    k_len_ = nblk_ = max_bn_ = max_bnp_ = 0;
     bn_.clear();
     start_.clear();
     koff_.clear();
     boff_.clear();
+    xoff_.clear();
+    base_len_ = xcols_ = 0;
     tiles_.clear();
     cap_N_ = cap_T_ = cap_kmul_ = 0;
     cap_percise_ = false;
-    sig_N_ = sig_T_ = 0;
+    sig_N_ = sig_T_ = sig_ch_ = 0;
+    sig_cap_ = 0;
+    d_sig_stage_ = nullptr;
     for (int c = 0; c < kLrMaxChannels; ++c) d_cap_[c] = d_sig_[c] = nullptr;
 }
 
@@ -105,47 +109,54 @@ int LearnRuntime::set_dense_blocks(int nblk, const float* const* data, const int
             return fail("set_dense_blocks_f32: K_len mismatch in block %d (%d vs %d)", b, k_len[b], kl);
     }
     try {
-        std::vector<float> kt1, kt2;
-        int start = 0;
+        int start = 0, ncol = 0;
         long long koff = 0, boff = 0;
+        std::vector<int> bnp, col_block;
+        for (int b = 0; b < nblk; ++b) ncol += bn[b];
         for (int b = 0; b < nblk; ++b) {
-            const int n = bn[b];
-            const size_t plane = static_cast<size_t>(n) * n;
+            const int n = bn[b], np = (n + 3) & ~3;
             bn_.push_back(n);
+            bnp.push_back(np);
             start_.push_back(start);
             koff_.push_back(koff);
             boff_.push_back(boff);
+            xoff_.push_back(static_cast<long long>(ncol) * xcols_);
+            col_block.insert(col_block.end(), n, b);
             max_bn_ = std::max(max_bn_, n);
-            kt1.resize(static_cast<size_t>(koff) + plane * kl);
-            kt2.resize(static_cast<size_t>(koff) + plane * kl);
-            // element K[i][j][tau] goes to kt1[tau][i][j] (base term) and, read as
-            // K_b[j'][k][tau] with j' = i, k = j, to kt2[tau][k][j'] (GEMM B operand)
-            const float* K = data[b];
-            for (int i = 0; i < n; ++i)
-                for (int j = 0; j < n; ++j)
-                    for (int tau = 0; tau < kl; ++tau) {
-                        const float v = K[(static_cast<size_t>(i) * n + j) * kl + tau];
-                        kt1[koff + tau * plane + static_cast<size_t>(i) * n + j] = v;
-                        kt2[koff + tau * plane + static_cast<size_t>(j) * n + i] = v;
-                    }
+            max_bnp_ = std::max(max_bnp_, np);
             start += n;
-            koff += static_cast<long long>(plane) * kl;
-            boff += static_cast<long long>(plane);
+            koff += static_cast<long long>(n) * np * kl;
+            boff += static_cast<long long>(n) * n;
+            xcols_ += np;
+        }
+        base_len_ = boff;
+        // element K[i][j][tau] goes to kp[tau][i][j], rows padded with zeros
+        std::vector<float> kp(static_cast<size_t>(koff), 0.f);
+        for (int b = 0; b < nblk; ++b) {
+            const int n = bn[b], np = bnp[b];
+            const size_t plane = static_cast<size_t>(n) * np;
+            for (int i = 0; i < n; ++i)
+                for (int tau = 0; tau < kl; ++tau) {
+                    const float* src = data[b] + static_cast<size_t>(i) * n * kl + tau;
+                    float* dst = kp.data() + koff_[b] + tau * plane + static_cast<size_t>(i) * np;
+                    for (int j = 0; j < n; ++j) dst[j] = src[static_cast<size_t>(j) * kl];
+                }
         }
         k_len_ = kl;
         nblk_ = nblk;
-        // column tile of the correction GEMM: 128 when a block is wider than 64
-        tile_cols_ = max_bn_ > 64 ? 128 : 64;
+        // column tile of the correction GEMM
+        tile_cols_ = max_bn_ > 64 ? 128 : max_bn_ > 32 ? 64 : 32;
         for (int b = 0; b < nblk; ++b)
             for (int j0 = 0; j0 < bn_[b]; j0 += tile_cols_) tiles_.push_back(make_int2(b, j0));
-        d_kt1_ = lupload(blk_mem_, kt1.data(), kt1.size());
-        d_kt2_ = lupload(blk_mem_, kt2.data(), kt2.size());
+        d_kp_ = lupload(blk_mem_, kp.data(), kp.size());
         d_koff_ = lupload(blk_mem_, koff_.data(), koff_.size());
         d_boff_ = lupload(blk_mem_, boff_.data(), boff_.size());
+        d_xoff_ = lupload(blk_mem_, xoff_.data(), xoff_.size());
         d_start_ = lupload(blk_mem_, start_.data(), start_.size());
         d_bn_ = lupload(blk_mem_, bn_.data(), bn_.size());
+        d_bnp_ = lupload(blk_mem_, bnp.data(), bnp.size());
+        d_col_block_ = lupload(blk_mem_, col_block.data(), col_block.size());
         d_tiles_ = lupload(blk_mem_, tiles_.data(), tiles_.size());
-        d_base_ = lalloc<float>(blk_mem_, static_cast<size_t>(boff));
     } catch (const std::exception& e) {
         clear_dense_blocks();
         return fail("set_dense_blocks_f32: %s", e.what());
@@ -253,18 +264,28 @@ void LearnRuntime::end_capture(float* out_vs_host, float* const* sig_host) {
 int LearnRuntime::load_signals(const float* it_nt, const float* dv_nt, const float* dp_nt, int N, int T,
                                bool percise) {
     try {
-        free_all(sig_mem_);
-        for (int c = 0; c < kLrMaxChannels; ++c) d_sig_[c] = nullptr;
+        // the buffers of the last call serve again where they are large enough (up to four
+        // times what is needed: a much smaller problem gives the memory back)
         const size_t n = static_cast<size_t>(N) * T;
-        float* stage = lalloc<float>(sig_mem_, n);
-        const float* src[3] = {it_nt, dv_nt, dp_nt};
         const int nch = percise ? 3 : 1;
-        for (int c = 0; c < nch; ++c) {
-            d_sig_[c] = lalloc<float>(sig_mem_, n);
-            LRC(hipMemcpy(stage, src[c], n * sizeof(float), hipMemcpyHostToDevice));
-            launch_transpose_nt_tn(stage, d_sig_[c], N, T, stream_);
-            LRC(hipStreamSynchronize(stream_));
+        if (sig_cap_ < n || sig_cap_ / 4 > n || sig_ch_ < nch) {
+            (void)hipStreamSynchronize(stream_);
+            free_all(sig_mem_);
+            sig_cap_ = 0;
+            sig_ch_ = 0;
+            for (int c = 0; c < kLrMaxChannels; ++c) d_sig_[c] = nullptr;
+            d_sig_stage_ = lalloc<float>(sig_mem_, n * nch);
+            for (int c = 0; c < nch; ++c) d_sig_[c] = lalloc<float>(sig_mem_, n);
+            sig_cap_ = n;
+            sig_ch_ = nch;
         }
+        const float* src[3] = {it_nt, dv_nt, dp_nt};
+        for (int c = 0; c < nch; ++c) {
+            float* stage = d_sig_stage_ + c * n;
+            LRC(hipMemcpyAsync(stage, src[c], n * sizeof(float), hipMemcpyHostToDevice, stream_));
+            launch_transpose_nt_tn(stage, d_sig_[c], N, T, stream_);
+        }
+        LRC(hipStreamSynchronize(stream_));    // the caller's arrays are read
         sig_N_ = N;
         sig_T_ = T;
     } catch (const std::exception& e) {
@@ -278,21 +299,20 @@ int LearnRuntime::replay(const ReplayIn& in) {
     const int T = in.source == SRC_CACHE ? cap_T_ : in.source == SRC_HOST ? sig_T_ : stream_T_;
     float* const* sig = in.source == SRC_CACHE ? d_cap_ : in.source == SRC_HOST ? d_sig_ : d_stream_;
     if (N <= 0 || T != in.ksteps + 1) return fail("replay: no signals of %d ticks", in.ksteps);
-    const int K_len = k_len_;
     const int ks = in.ksteps;
     try {
-        // workspace: history ring, base scratch, per-tick vectors, norm partials
-        const int R = in.percise ? K_len + 1 : 1;
-        const size_t slice = static_cast<size_t>(N) * N;
-        const int ntiles = static_cast<int>(tiles_.size());
-        const int nwg = ntiles * rp_corr_row_tiles(N);
-        const std::vector<long long> key = {N, R, ks, in.n_out, in.n_in, nwg, in.percise ? 1 : 0};
+        const Sizes z = sizes_for(N, in.percise);
+        const std::vector<long long> key = {N, z.R, ks, in.n_out, in.n_in, in.percise ? 1 : 0};
         if (key != ws_key_) {
             free_all(ws_mem_);
             ws_key_.clear();
-            ws_.hist = lalloc<float>(ws_mem_, slice * R);
-            ws_.ghist = in.percise ? lalloc<float>(ws_mem_, slice * R) : nullptr;
-            ws_.slot_scale = lalloc<float>(ws_mem_, R);
+            const size_t slice = static_cast<size_t>(N) * N;
+            ws_.slices = lalloc<float>(ws_mem_, 2 * slice);
+            ws_.x = lalloc<float>(ws_mem_, z.x);
+            ws_.part = lalloc<float>(ws_mem_, z.part);
+            ws_.base_ticks = kBaseTicks;
+            ws_.base = lalloc<float>(ws_mem_, static_cast<size_t>(base_len_) * kBaseTicks);
+            ws_.slot_scale = lalloc<float>(ws_mem_, z.R);
             ws_.gs = lalloc<float>(ws_mem_, 1);
             ws_.tick_scale = lalloc<float>(ws_mem_, 1);
             ws_.w_tick = lalloc<float>(ws_mem_, N);
@@ -302,9 +322,10 @@ int LearnRuntime::replay(const ReplayIn& in) {
             ws_.pre = lalloc<int>(ws_mem_, N);
             ws_.pin = lalloc<int>(ws_mem_, std::max(in.n_in, 1));
             ws_.dx = lalloc<float>(ws_mem_, static_cast<size_t>(std::max(in.n_in, 1)) * ks);
-            ws_.norm_part = lalloc<double>(ws_mem_, nwg);
-            ws_.flag_part = lalloc<int>(ws_mem_, nwg);
+            ws_.norm_part = lalloc<double>(ws_mem_, z.norm);
             ws_.dw_out = lalloc<float>(ws_mem_, N);
+            // the padding of the X rows stays zero: only the columns themselves are written
+            if (z.x) launch_fill_f32(ws_.x, 0.f, static_cast<long long>(z.x), stream_);
             ws_key_ = key;
         }
     } catch (const std::exception& e) {
@@ -313,6 +334,20 @@ int LearnRuntime::replay(const ReplayIn& in) {
         return fail("replay: %s", e.what());
     }
     return replay_on(in, ws_, sig, N);
+}
+
+LearnRuntime::Sizes LearnRuntime::sizes_for(int N, bool percise) const {
+    Sizes z;
+    const int row_tiles = rp_corr_row_tiles(N);
+    const int ntiles = static_cast<int>(tiles_.size());
+    z.R = percise ? k_len_ + 1 : 1;
+    z.norm = static_cast<size_t>(std::max(ntiles * row_tiles, rp_finish_blocks(N)));
+    if (percise) {
+        const int splits = rp_corr_splits(N, ntiles, max_bnp_, k_len_);   // the most any window takes
+        z.x = static_cast<size_t>(z.R) * N * xcols_;
+        z.part = splits > 1 ? static_cast<size_t>(splits) * N * N : 0;
+    }
+    return z;
 }
 
 // The replay proper over signals sig[c] ((T, N) on the device) with the buffers of ws;
@@ -324,36 +359,21 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
     try {
         const int R = in.percise ? K_len + 1 : 1;
         const size_t slice = static_cast<size_t>(N) * N;
+        const long long xslice = static_cast<long long>(N) * xcols_;
         const int ntiles = static_cast<int>(tiles_.size());
-        const int nwg = ntiles * rp_corr_row_tiles(N);
-        float* hist = ws.hist;
-        float* ghist = ws.ghist;
-        float* slot_scale = ws.slot_scale;
-        float* gs = ws.gs;
-        float* tick_scale = ws.tick_scale;
-        float* w_tick = ws.w_tick;
-        float* dw_acc = ws.dw_acc;
-        float* dl = ws.dl;
-        int* po = ws.po;
-        int* pre = ws.pre;
-        int* pin = ws.pin;
-        float* dx = ws.dx;
-        double* norm_part = ws.norm_part;
-        int* flag_part = ws.flag_part;
-        float* dw_out = ws.dw_out;
-        LRC(hipMemcpyAsync(dl, in.dl, sizeof(float) * static_cast<size_t>(ks) * in.n_out, hipMemcpyHostToDevice,
+        const int row_tiles = rp_corr_row_tiles(N);
+        LRC(hipMemcpyAsync(ws.dl, in.dl, sizeof(float) * static_cast<size_t>(ks) * in.n_out, hipMemcpyHostToDevice,
                            stream_));
-        LRC(hipMemcpyAsync(po, in.po, sizeof(int) * in.n_out, hipMemcpyHostToDevice, stream_));
-        LRC(hipMemcpyAsync(pre, in.pre, sizeof(int) * N, hipMemcpyHostToDevice, stream_));
-        if (need_dx) LRC(hipMemcpyAsync(pin, in.pin, sizeof(int) * in.n_in, hipMemcpyHostToDevice, stream_));
+        LRC(hipMemcpyAsync(ws.po, in.po, sizeof(int) * in.n_out, hipMemcpyHostToDevice, stream_));
+        LRC(hipMemcpyAsync(ws.pre, in.pre, sizeof(int) * N, hipMemcpyHostToDevice, stream_));
+        if (need_dx) LRC(hipMemcpyAsync(ws.pin, in.pin, sizeof(int) * in.n_in, hipMemcpyHostToDevice, stream_));
 
-        launch_fill_f32(hist, 0.f, static_cast<long long>(slice), stream_);      // slot 0: tick 0
-        if (in.percise) launch_fill_f32(ghist, 0.f, static_cast<long long>(slice), stream_);
-        launch_fill_f32(slot_scale, 1.f, R, stream_);
-        launch_fill_f32(gs, static_cast<float>(in.grad_scale), 1, stream_);
-        launch_fill_f32(tick_scale, 1.f, 1, stream_);
-        launch_fill_f32(dw_acc, 0.f, N, stream_);
-        if (need_dx) launch_fill_f32(dx, 0.f, static_cast<long long>(in.n_in) * ks, stream_);
+        launch_fill_f32(ws.slices, 0.f, static_cast<long long>(slice), stream_);      // tick 0
+        launch_fill_f32(ws.slot_scale, 1.f, R, stream_);
+        launch_fill_f32(ws.gs, static_cast<float>(in.grad_scale), 1, stream_);
+        launch_fill_f32(ws.tick_scale, 1.f, 1, stream_);
+        launch_fill_f32(ws.dw_acc, 0.f, N, stream_);
+        if (need_dx) launch_fill_f32(ws.dx, 0.f, static_cast<long long>(in.n_in) * ks, stream_);
 
         const float dt = static_cast<float>(in.dt);
         const float eps = static_cast<float>(in.eps);
@@ -362,83 +382,144 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
         corr_launches = 0;
         std::vector<std::pair<hipEvent_t, hipEvent_t>> evs;
 
+        ReplayTickArgs K{};
+        K.N = N;
+        K.norm_part = ws.norm_part;
+        K.thr = thr;
+        K.gs = ws.gs;
+        K.slot_scale = ws.slot_scale;
+        K.R = R;
+        K.tick_scale = ws.tick_scale;
+        K.po = ws.po;
+        K.n_out = in.n_out;
+        K.w_tick = ws.w_tick;
+        K.dw_acc = ws.dw_acc;
+        K.xoff = d_xoff_;
+        K.col_block = d_col_block_;
+        K.start = d_start_;
+        K.bnp = d_bnp_;
+        K.pre = ws.pre;
+        // X of tick t (from slice `cur` into its slot), read by the ticks after it
+        auto with_x = [&](int t) {
+            const bool need = in.percise && t < ks;
+            K.x = need ? ws.x + static_cast<size_t>(t % R) * xslice : nullptr;
+            K.dv = need ? sig[1] + static_cast<size_t>(t + 1) * N : nullptr;
+            K.dp = need ? sig[2] + static_cast<size_t>(t + 1) * N : nullptr;
+        };
+        K.cur = ws.slices;
+        K.dl = nullptr;
+        with_x(0);
+        launch_rp_tick(K, stream_);
+
+        ReplayDx X{};                     // dx of the tick before (none at the first)
+        X.pin = ws.pin;
+        X.w_tick = ws.w_tick;
+        X.eps = eps;
+        X.ksteps = ks;
+        X.tick_scale = ws.tick_scale;
+        X.dx = ws.dx;
+
+        ReplayOut O{};
+        O.N = N;
+        O.dt = dt;
+        O.gs = ws.gs;
+        O.norm_part = ws.norm_part;
+
         for (int t_lr = 1; t_lr <= ks; ++t_lr) {
             const int tw = std::min(t_lr, K_len);
-            const int it_t0 = t_lr - tw + 1;
-            const int k_t0 = K_len - tw;
             const int cur = in.percise ? t_lr % R : 0;
-            float* out = hist + static_cast<size_t>(cur) * slice;
             bool due = false;
             if (in.clip_strategy != 0) {
                 if (in.cached_clip_rule) due = in.clip_strategy == 1 || (t_lr % in.clip_every) == 0;
                 else due = in.clip_strategy == 1 && (t_lr % in.clip_every) == 0;
             }
 
-            ReplayBaseArgs B{};
-            B.kt1 = d_kt1_;
-            B.koff = d_koff_;
-            B.boff = d_boff_;
-            B.start = d_start_;
-            B.bn = d_bn_;
-            B.it = sig[0];
-            B.N = N;
-            B.it_t0 = it_t0;
-            B.k_t0 = k_t0;
-            B.tw = tw;
-            B.dt = dt;
-            B.gs = gs;
-            B.base = d_base_;
-            B.slot_scale = slot_scale;
-            B.cur = cur;
-            launch_rp_base(B, nblk_, max_bn_, stream_);
-
-            ReplayCorrArgs C{};
-            C.hist = hist;
-            C.ghist = ghist;
-            C.slice = static_cast<long long>(slice);
-            C.slot_scale = slot_scale;
-            C.R = R;
-            C.dv = sig[1];
-            C.dp = sig[2];
-            C.pre = pre;
-            C.kt2 = d_kt2_;
-            C.koff = d_koff_;
-            C.start = d_start_;
-            C.bn = d_bn_;
-            C.base = d_base_;
-            C.boff = d_boff_;
-            C.tiles = d_tiles_;
-            C.N = N;
-            C.t_lr = t_lr;
-            C.tw = in.percise ? tw : 0;
-            C.it_t0 = it_t0;
-            C.k_t0 = k_t0;
-            C.dt = dt;
-            C.out = out;
-            C.sanitize = due ? 1 : 0;
-            C.norm_part = norm_part;
-            C.flag_part = flag_part;
-            if (timing) {
-                hipEvent_t a, b;
-                LRC(hipEventCreate(&a));
-                LRC(hipEventCreate(&b));
-                LRC(hipEventRecord(a, stream_));
-                launch_rp_corr(C, ntiles, tile_cols_, stream_);
-                LRC(hipEventRecord(b, stream_));
-                evs.push_back({a, b});
-            } else {
-                launch_rp_corr(C, ntiles, tile_cols_, stream_);
+            const int bt = (t_lr - 1) % ws.base_ticks;
+            if (bt == 0) {
+                ReplayBaseArgs B{};
+                B.kp = d_kp_;
+                B.koff = d_koff_;
+                B.boff = d_boff_;
+                B.start = d_start_;
+                B.bn = d_bn_;
+                B.bnp = d_bnp_;
+                B.it = sig[0];
+                B.N = N;
+                B.T = ks + 1;
+                B.K_len = K_len;
+                B.t0 = t_lr;
+                B.ng = std::min(ws.base_ticks, ks - t_lr + 1);
+                B.base = ws.base;
+                B.base_stride = base_len_;
+                launch_rp_base(B, nblk_, max_bn_, stream_);
             }
-            if (in.percise) launch_rp_pregather(out, pre, N, ghist + static_cast<size_t>(cur) * slice, stream_);
-            if (due) launch_rp_clip(norm_part, flag_part, nwg, thr, gs, slot_scale, R, tick_scale, stream_);
-            launch_rp_wtick(out, slot_scale, cur, N, po, in.n_out, dl + static_cast<size_t>(t_lr - 1) * in.n_out,
-                            due ? 1 : 0, tick_scale, w_tick, dw_acc, stream_);
-            if (need_dx)
-                launch_rp_dx(out, slot_scale, cur, N, pin, in.n_in, w_tick, eps, t_lr - 1, ks, due ? 1 : 0,
-                             tick_scale, dx, stream_);
+            O.base = ws.base + static_cast<size_t>(bt) * base_len_;
+            O.out = ws.slices + static_cast<size_t>(t_lr & 1) * slice;
+            O.sanitize = due ? 1 : 0;
+
+            const int nsplit = in.percise ? rp_corr_splits(N, ntiles, max_bnp_, tw) : 0;
+            if (in.percise) {
+                ReplayCorrArgs C{};
+                C.x = ws.x;
+                C.xslice = xslice;
+                C.xoff = d_xoff_;
+                C.slot_scale = ws.slot_scale;
+                C.R = R;
+                C.h0 = (t_lr - tw) % R;
+                C.kp = d_kp_;
+                C.koff = d_koff_;
+                C.start = d_start_;
+                C.bn = d_bn_;
+                C.bnp = d_bnp_;
+                C.boff = d_boff_;
+                C.tiles = d_tiles_;
+                C.row_tiles = row_tiles;
+                C.nsplit = nsplit;
+                C.ncorr = ntiles * row_tiles * nsplit;
+                C.tw = tw;
+                C.k_t0 = K_len - tw;
+                C.part = ws.part;
+                C.O = O;
+                if (nsplit == 1) C.dx = X;
+                if (timing) {
+                    hipEvent_t a, b;
+                    LRC(hipEventCreate(&a));
+                    LRC(hipEventCreate(&b));
+                    LRC(hipEventRecord(a, stream_));
+                    launch_rp_corr(C, tile_cols_, stream_);
+                    LRC(hipEventRecord(b, stream_));
+                    evs.push_back({a, b});
+                } else {
+                    launch_rp_corr(C, tile_cols_, stream_);
+                }
+            }
+            if (nsplit != 1) {
+                ReplayFinishArgs F{};
+                F.part = ws.part;
+                F.nsplit = nsplit;
+                F.col_block = d_col_block_;
+                F.start = d_start_;
+                F.bn = d_bn_;
+                F.boff = d_boff_;
+                F.O = O;
+                F.dx = X;
+                launch_rp_finish(F, stream_);
+            }
+            K.cur = O.out;
+            K.due = due ? 1 : 0;
+            K.npart = nsplit == 1 ? ntiles * row_tiles : rp_finish_blocks(N);
+            K.cur_slot = cur;
+            K.dl = ws.dl + static_cast<size_t>(t_lr - 1) * in.n_out;
+            with_x(t_lr);
+            launch_rp_tick(K, stream_);
+            X.n_in = in.n_in;
+            X.cur = O.out;
+            X.t_idx = t_lr - 1;
+            X.clip_ran = due ? 1 : 0;
         }
+        launch_rp_dx(X, N, stream_);
         // dw = dw_accum * (1 / ksteps) in fp32 (LearnRuntime.cpp:2281-2285)
-        launch_rp_scale_into(dw_acc, 1.0f / static_cast<float>(ks), dw_out, N, stream_);
+        launch_rp_scale_into(ws.dw_acc, 1.0f / static_cast<float>(ks), ws.dw_out, N, stream_);
         LRC(hipStreamSynchronize(stream_));
         LRC(hipGetLastError());
         for (auto& pr : evs) {
@@ -449,9 +530,9 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
             (void)hipEventDestroy(pr.first);
             (void)hipEventDestroy(pr.second);
         }
-        LRC(hipMemcpy(in.dw_out, dw_out, sizeof(float) * N, hipMemcpyDeviceToHost));
+        LRC(hipMemcpy(in.dw_out, ws.dw_out, sizeof(float) * N, hipMemcpyDeviceToHost));
         if (need_dx)
-            LRC(hipMemcpy(in.dx_out, dx, sizeof(float) * static_cast<size_t>(in.n_in) * ks, hipMemcpyDeviceToHost));
+            LRC(hipMemcpy(in.dx_out, ws.dx, sizeof(float) * static_cast<size_t>(in.n_in) * ks, hipMemcpyDeviceToHost));
     } catch (const std::exception& e) {
         return fail("replay: %s", e.what());
     }
@@ -505,17 +586,42 @@ int LearnRuntime::replay_from_host_noalloc(const ReplayIn& in, const float* it_n
     if (N <= 0 || T != in.ksteps + 1) return fail("replay: no signals of %d ticks", in.ksteps);
     try {
         const int nch = in.percise ? 3 : 1;
-        const int R = in.percise ? k_len_ + 1 : 1;
+        const Sizes z = sizes_for(N, in.percise);
         const size_t slice = static_cast<size_t>(N) * N;
         const size_t sigsz = static_cast<size_t>(N) * T;
-        const int nwg = static_cast<int>(tiles_.size()) * rp_corr_row_tiles(N);
         const int ks = in.ksteps;
-        auto carve = [&](Carver& c, Workspace& w, float** sig, float** stage) {
-            *stage = c.take<float>(sigsz);
+        // what is refused: two rings of slices (one without the precise term), the signals
+        // and the vectors past the limit
+        const size_t nwg = static_cast<size_t>(tiles_.size()) * rp_corr_row_tiles(N);
+        Carver measure{nullptr};
+        for (int ch = 0; ch <= nch; ++ch) measure.take<float>(sigsz);
+        for (int ring = 0; ring < (in.percise ? 2 : 1); ++ring) measure.take<float>(slice * z.R);
+        for (size_t n : {static_cast<size_t>(z.R), static_cast<size_t>(1), static_cast<size_t>(1),
+                         static_cast<size_t>(N), static_cast<size_t>(N), static_cast<size_t>(ks) * in.n_out,
+                         static_cast<size_t>(in.n_out), static_cast<size_t>(N),
+                         static_cast<size_t>(std::max(in.n_in, 1)), static_cast<size_t>(std::max(in.n_in, 1)) * ks})
+            measure.take<float>(n);
+        measure.take<double>(nwg);
+        measure.take<int>(nwg);
+        measure.take<float>(N);
+        if (measure.used > kNoAllocLimitBytes)
+            return fail("replay needs %zu bytes of device scratch for N=%d, T=%d, K_len=%d%s; the allocation-free "
+                        "entry point holds at most %zu bytes (use the allocating one)",
+                        measure.used, N, T, k_len_, in.percise ? " (percise)" : "", kNoAllocLimitBytes);
+        Workspace w;
+        float* sig[kLrMaxChannels];
+        float* stage = nullptr;
+        // as many ticks' base terms as there is room for (they are made a few ticks at a
+        // time; how many changes no result)
+        auto carve = [&](Carver& c, int base_ticks) {
+            stage = c.take<float>(sigsz);
             for (int ch = 0; ch < kLrMaxChannels; ++ch) sig[ch] = ch < nch ? c.take<float>(sigsz) : nullptr;
-            w.hist = c.take<float>(slice * R);
-            w.ghist = in.percise ? c.take<float>(slice * R) : nullptr;
-            w.slot_scale = c.take<float>(R);
+            w.slices = c.take<float>(2 * slice);
+            w.x = c.take<float>(z.x);
+            w.part = c.take<float>(z.part);
+            w.base_ticks = base_ticks;
+            w.base = c.take<float>(static_cast<size_t>(base_len_) * base_ticks);
+            w.slot_scale = c.take<float>(z.R);
             w.gs = c.take<float>(1);
             w.tick_scale = c.take<float>(1);
             w.w_tick = c.take<float>(N);
@@ -525,21 +631,19 @@ int LearnRuntime::replay_from_host_noalloc(const ReplayIn& in, const float* it_n
             w.pre = c.take<int>(N);
             w.pin = c.take<int>(std::max(in.n_in, 1));
             w.dx = c.take<float>(static_cast<size_t>(std::max(in.n_in, 1)) * ks);
-            w.norm_part = c.take<double>(nwg);
-            w.flag_part = c.take<int>(nwg);
+            w.norm_part = c.take<double>(z.norm);
             w.dw_out = c.take<float>(N);
+            return c.used;
         };
-        Workspace w;
-        float* sig[kLrMaxChannels];
-        float* stage = nullptr;
-        Carver measure{nullptr};
-        carve(measure, w, sig, &stage);
-        if (measure.used > kNoAllocScratchBytes)
-            return fail("replay needs %zu bytes of device scratch for N=%d, T=%d, K_len=%d%s; the allocation-free "
-                        "entry point holds at most %zu bytes (use the allocating one)",
-                        measure.used, N, T, k_len_, in.percise ? " (percise)" : "", kNoAllocScratchBytes);
+        int base_ticks = kBaseTicks;
+        for (;; base_ticks /= 2) {
+            Carver probe{nullptr};
+            if (carve(probe, base_ticks) <= kNoAllocScratchBytes) break;
+            if (base_ticks == 1) return fail("replay: the scratch array is too small for N=%d, T=%d", N, T);
+        }
         Carver c{noalloc_scratch()};
-        carve(c, w, sig, &stage);
+        carve(c, base_ticks);
+        if (z.x) launch_fill_f32(w.x, 0.f, static_cast<long long>(z.x), stream_);
         // (N, T) host signals -> (T, N) on the device, as load_signals does
         const float* src[kLrMaxChannels] = {it_nt, dv_nt, dp_nt};
         for (int ch = 0; ch < nch; ++ch) {

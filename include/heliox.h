@@ -448,11 +448,11 @@ int hx_replay_compute_dw_dx_from_signals_into(hx_sim* sim, const float* it_lr_nt
  * forbid hipMalloc).  It cannot be captured into a HIP graph: it copies the host signals in
  * and the results back synchronously and synchronises the library's stream before it
  * returns.  Same arguments, checks and results;
- * every device buffer (the signals, the dv/dw history ring, the per-tick vectors) is
- * carved from one fixed 64 MiB device array that the library holds on each GPU it runs
- * on until the process ends, so the call makes no hipMalloc/hipFree.  A problem whose
- * buffers do not fit (about 8 (K_len + 1) N^2 + 16 N T bytes with percise) is refused
- * with an error.  The dense blocks must already be set.  Every call on one GPU shares
+ * every device buffer (the signals, the history ring, the per-tick vectors) is carved
+ * from one fixed 256 MiB device array that the library holds on each GPU it runs on until
+ * the process ends, so the call makes no hipMalloc/hipFree.  A problem of more than 64 MiB
+ * of signals, history and vectors (about 8 (K_len + 1) N^2 + 16 N T bytes with percise) is
+ * refused with an error.  The dense blocks must already be set.  Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (from several threads) race. */
 int hx_replay_compute_dw_dx_from_signals_into_noalloc(
     hx_sim* sim, const float* it_lr_nt, const float* ditdv_lr_nt, const float* ditdvpre_lr_nt, int N, int T,

@@ -1,0 +1,71 @@
+"""The replay's correction GEMM at the edges of its tiles and splits, against the oracle:
+column tiles of 32, 64 and 128 and one more or less, rows that do not fill a 128-row tile,
+block widths that are not a multiple of 4 (padded rows), reductions of one chunk, of a few
+(one per split) and of many, several taps per chunk, more ticks than one launch of the base
+term makes, and an infinite signal on clip ticks.
+
+An entry of dv/dw is an fp32 sum of m = K_len (bn + 1) products whose rounding errors add
+up like a random walk, sqrt(m) 2^-24 of the largest partial sum; the bound allows sixteen
+times that, relative to the largest result."""
+import numpy as np
+import pytest
+
+from heliox_amd import Sim, build_config
+from oracle import lrds
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sim(gpu_lib):
+    g = Sim()
+    g.load_model_from_spec(build_config(1, 1, 10.0))
+    return g
+
+
+CASES = [
+    # bns, K_len, ksteps, percise, thr, infinite signal
+    ((1,), 1, 3, True, 1e6, False),
+    ((1, 2, 3), 4, 10, True, 1e6, False),
+    ((31,), 2, 9, True, 1e6, False),
+    ((32, 32), 3, 8, True, 0.05, False),
+    ((33, 30), 2, 17, True, 1e6, False),
+    ((63, 65), 2, 6, True, 1e6, False),
+    ((127, 2), 1, 5, True, 1e6, False),
+    ((128, 128, 1), 2, 9, True, 1e6, False),
+    ((130,), 3, 7, True, 1e6, False),
+    ((5,) * 40, 16, 25, True, 0.5, False),
+    ((16, 17), 64, 70, True, 1e6, False),
+    ((70, 58), 6, 19, False, 0.05, False),
+    ((40, 23), 5, 12, True, 1.0, True),
+]
+
+
+@pytest.mark.parametrize("bns,K_len,ksteps,percise,thr,inf", CASES)
+def test_replay_at_tile_edges_matches_oracle(sim, bns, K_len, ksteps, percise, thr, inf):
+    print(f"case lrds tiles bns={bns[:3]}x{len(bns)} K_len={K_len} ksteps={ksteps} percise={percise} thr={thr}",
+          flush=True)
+    rng = np.random.default_rng(len(bns) * 1000 + bns[0] + K_len)
+    N, T = int(sum(bns)), ksteps + 1
+    blocks = [(rng.normal(0, 1, (bn, bn, K_len)) * 0.3 / np.sqrt(bn)).astype(np.float32) for bn in bns]
+    it, dv, dp = (rng.normal(0, s, (N, T)).astype(np.float32) for s in (1.0, 0.3, 0.3))
+    if inf:
+        dv[3, 4] = np.inf
+    pre = np.where(rng.random(N) < 0.6, rng.integers(0, N, N), -1).astype(np.int32)
+    po = np.sort(rng.choice(N, min(N, 9), replace=False)).astype(np.int32)
+    pin = np.sort(rng.choice(N, min(N, 3), replace=False)).astype(np.int32)
+    dL = rng.normal(0, 1, (ksteps, po.size)).astype(np.float32)
+    assert sim.set_dense_blocks_f32(blocks) == K_len
+    dw, dx = np.zeros(N, np.float32), np.zeros((pin.size, ksteps), np.float32)
+    rc = sim.replay_compute_dw_dx_from_signals_into(it, dv, dp, dL, po, pin, pre, dw, dx, 0.1, percise, grad_scale=1.3,
+                                                    eps=4.0, grad_l2norm_threshold=thr)
+    assert rc == 0, sim.last_error()
+    with np.errstate(all="ignore"):
+        rdw, rdx, _ = lrds.replay(it, dv, dp, blocks, dL, po, pre, dt=0.1, percise=percise, pinput=pin, grad_scale=1.3,
+                                  eps=4.0, grad_l2norm_threshold=thr, clip_strategy=1, variant="signals")
+    assert np.all(np.isfinite(rdw)) and np.all(np.isfinite(rdx))
+    tol = 16 * np.sqrt(K_len * (max(bns) + 1)) * 2.0 ** -24
+    for name, a, r in (("dw", dw, rdw), ("dx", dx, rdx)):
+        err, scale = float(np.max(np.abs(a - r))), float(np.max(np.abs(r)))
+        print(f"  {name} max err {err:.3e} scale {scale:.3e} tol {tol:.1e}", flush=True)
+        assert err <= tol * scale + 1e-9
