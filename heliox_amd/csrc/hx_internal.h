@@ -194,6 +194,50 @@ struct SolveArgs {
     int res_rounds;               //   and this many rounds (the largest unit's); 0: rounds streamed from HBM
 };
 
+// Solve by substructuring (k_solve_split): a pack is a run of a unit's cells, one workgroup
+// of one thread per chunk.  Its slots are the breadth-first order of its chunks, so the
+// chunks of one tree level are consecutive and so are those hanging off one tail; its
+// threads follow the unit's rounds, so that neighbouring threads read neighbouring nodes.
+struct alignas(16) SplitDesc {
+    int base;              // solver-order node of the chunk's head
+    int round;             // its round (in all rounds): node k sits at base + off[k] - off[0]
+    uint16_t slot;         // pack-local; kNone: a thread without a chunk
+    uint16_t parent;       // slot of the chunk whose tail is the head's parent (kNone: root)
+    uint16_t child_begin;  // slots of the chunks hanging off the tail
+    uint8_t len;
+    uint8_t child_count;
+};
+static_assert(sizeof(SplitDesc) == 16, "SplitDesc must stay 16 bytes");
+// A cell of more chunks (three wavefronts a SIMD at 168 registers) is left to the round-by-round solve; a
+// pack stops taking cells at kSplitPackChunks (two wavefronts).
+constexpr int kSplitMaxChunks = 768;
+constexpr int kSplitPackChunks = 128;
+// The chunks the chip holds at once (256 CUs, 12 wavefronts of this kernel's registers).  A
+// model of more has workgroups queueing, and the rounds, which leave room for the other
+// group's node pass beside them, catch up: for cells whose rounds are held in LDS at about
+// this many (100 steps of 500-node trees: 1500 cells, 80k chunks, 10.4 -> 7.7 ms; 3000,
+// 161k, 12.8 -> 11.8; 6000, 322k, 22.3 -> 25.6), for larger, streamed cells past twice as
+// many (5000-node pyramidal cells: 300, 185k, 19.0 -> 12.8 ms; 600, 371k, 28.8 -> 25.6;
+// 1000, 619k, even; 2000, 1.24M, 0.52 -> 0.64 ms a step).  A rule on the model's chunks and
+// largest cell, not its packs, so that no choice of units or groups changes the route.
+constexpr long long kSplitMaxTotal = 256LL * 12 * kWave;
+struct SplitArgs {
+    const SplitDesc* desc;        // [npack * threads]
+    const int* levels;            // [npack * lev_stride]: level count, then the first slot of each level and the end
+    int threads;                  // workgroup size, a multiple of the wavefront
+    int lev_stride;
+    int npack;
+    double* vold;                 // when store_vold: the voltages before the solve
+    int store_vold;
+    int yform;                    // as SolveArgs
+    const RoundInfo* rounds;
+    double* v;
+    const double* d;              // neither d nor rhs is written
+    const double* rhs;
+    const double* a;
+    const double* b;
+};
+
 // Event ring: one slot per delivery step (mod nslot), fixed capacity per slot.
 struct EventRing {
     int* count;                   // [nslot]
@@ -551,6 +595,7 @@ void launch_after_solve(AfterSolve p, hipStream_t s);
 void launch_point_state(int mech, const StepArgs& a, hipStream_t s);
 void launch_init(int mech, const StepArgs& a, hipStream_t s);
 void launch_set_v(double* v, int n, double val, hipStream_t s);
+void launch_solve_split(const SplitArgs& a, hipStream_t s);
 void launch_solve(const SolveArgs& a, int max_chunks, hipStream_t s);
 void launch_input_set(const InputSet& a, hipStream_t s);
 void launch_deliver_set(const DeliverArgs& a, const RingSet& rings, int nblk, hipStream_t s);

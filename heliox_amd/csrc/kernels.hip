@@ -19,6 +19,8 @@
 //                    substitution and v update; junction values through LDS
 //   k_solve_res .... the same for units small enough to be held whole in LDS:
 //                    read once, solved in LDS records, written once
+//   k_solve_split .. one thread per chunk: chunk interiors at once, then the tree
+//                    of the chunks' tails (most models; the two above otherwise)
 //   k_spike ........ threshold detection, wave-ballot compaction into the spike
 //                    log, fan-out of deliveries into the device event ring
 //   k_input ........ VecStim trains (sorted on the host) entering the ring;
@@ -1259,6 +1261,236 @@ __global__ void __launch_bounds__(kWave * kSolveMaxWaves) k_solve_res(SolveArgs 
 }
 
 // ---------------------------------------------------------------------------
+// tree solve by substructuring
+// ---------------------------------------------------------------------------
+// The round-by-round solve walks a chain of dependent 16-node chunks (26 rounds each way
+// for a 5000-compartment pyramidal cell) on one wavefront, about 2 us a round.  Here every
+// chunk eliminates its own interior (all nodes but its tail, from the head on) at once, one
+// thread per chunk: an interior row keeps one fill column, the tail of the parent chunk p,
+//   D_k x_k + a_{k+1} x_{k+1} + F_k x_p = R_k,    row p gains E_k x_k,
+// and what remains is a tree over the tails alone, one node per chunk, solved level by level
+// on one wavefront; then every chunk substitutes its interior from x_p and its tail at once:
+//   x_k = u_k - w_k x_{k+1} - f_k x_p.
+// The serial chain is one chunk plus a short step per level instead of a whole chunk per
+// round, and u, w and f stay in registers: a node is read once (d, rhs, a, b, v) and
+// written once (v), 48 bytes (40 with kY) where the streamed rounds move 80 (72).
+// Which unit or pack a cell sits in changes no arithmetic, so the bits do not depend on it.
+// d and rhs keep the assembled matrix; the pivots and x that the reference leaves there
+// come from the round-by-round solve when something reads them.  Bound by latency: the dependent loads
+// (descriptor, round, node), one chunk's chain and the levels.
+// Measured figures: a 101-node cell k_solve_res 18 us, 500-node trees 30 us, 5000-node
+// pyramidal cells k_solve 87 us (10 cells); this kernel 13, 15 and 23 us.
+//
+// kY: rhs holds rhs + d v and the unknown is the new voltage, v is not read (but for kX);
+// otherwise the unknown is its change, with the axial terms as differences of voltages.
+// kX: the old voltages go to vold.
+constexpr int kSplitFields = 6;
+struct SplitTail {
+    double D, R, E, F, dp, rp;
+    int kids;                // first child slot, child count in the upper half
+};
+enum SplitField { SF_D, SF_R, SF_E, SF_F, SF_DP, SF_RP };
+inline size_t split_lds_bytes(int threads, int lev_stride) {
+    return static_cast<size_t>(threads) * (sizeof(double) * (kSplitFields + 1) + 2 * sizeof(int)) +
+           sizeof(int) * lev_stride;
+}
+// kT: the largest workgroup.  Up to 512 threads nothing spills; the change form at 768 (168
+// registers a thread) spills 34 of them, the voltage form none.
+template <int kX, int kY, int kT>
+__global__ void __launch_bounds__(kT) k_solve_split(SplitArgs S) {
+    extern __shared__ double lds[];
+    const int nt = S.threads;
+    const int t = static_cast<int>(threadIdx.x);
+    double* rec = lds;                          // [kSplitFields][nt], by slot
+    double* xt = lds + kSplitFields * nt;       // tail values: v before the solve, then x
+    int* kids = reinterpret_cast<int*>(xt + nt);
+    int* par = kids + nt;
+    int* lev = par + nt;
+    const SplitDesc q = S.desc[static_cast<size_t>(blockIdx.x) * nt + t];
+    for (int i = t; i < S.lev_stride; i += nt) lev[i] = S.levels[static_cast<size_t>(blockIdx.x) * S.lev_stride + i];
+    const bool act = q.slot != kNone;
+    const bool root = q.parent == kNone;
+    const int len = act ? q.len : 0;
+    const RoundV rv = load_round(S.rounds, q.round);
+    const uint32_t off[kChunk / 2] = {rv.x0.z, rv.x0.w, rv.x1.x, rv.x1.y, rv.x1.z, rv.x1.w, rv.x2.x, rv.x2.y};
+    // node k of the chunk; past its end, the head again (every load stays in the model)
+    auto at = [&](int k) { return q.base + (k < len ? static_cast<int>((off[k >> 1] >> (16 * (k & 1))) & 0xFFFF) : 0); };
+    int wlen = kChunk;                          // the wavefront's longest chunk, by quarters
+    if (!__any(len > 12)) wlen = 12;
+    if (!__any(len > 8)) wlen = 8;
+    if (!__any(len > 4)) wlen = 4;
+    double dk[kChunk], rk[kChunk], ak[kChunk], bk[kChunk], vk[kY ? 1 : kChunk];
+#pragma unroll
+    for (int g = 0; g < kChunk; g += 4) {
+        if (g < wlen) {
+#pragma unroll
+            for (int k = g; k < g + 4; ++k) {
+                const int i = at(k);
+                dk[k] = S.d[i];
+                rk[k] = S.rhs[i];
+                ak[k] = S.a[i];
+                bk[k] = S.b[i];
+                if constexpr (!kY) vk[k] = S.v[i];
+            }
+        } else {
+#pragma unroll
+            for (int k = g; k < g + 4; ++k) {
+                dk[k] = rk[k] = ak[k] = bk[k] = 0.0;
+                if constexpr (!kY) vk[k] = 0.0;
+            }
+        }
+    }
+    if (act) {
+        kids[q.slot] = q.child_begin | (static_cast<int>(q.child_count) << 16);
+        par[q.slot] = q.parent;
+    }
+    if (root) ak[0] = bk[0] = 0.0;
+    double dvp = 0.0;                           // v_p - v_head
+    if constexpr (!kY) {
+        double vt = vk[0];
+#pragma unroll
+        for (int k = 1; k < kChunk; ++k)
+            if (k == len - 1) vt = vk[k];
+        if (act) xt[q.slot] = vt;
+        __syncthreads();
+        if (act && !root) dvp = xt[q.parent] - vk[0];
+    }
+    // interior elimination, head to tail
+    double D = dk[0] - bk[0], R = rk[0], F = bk[0], E = ak[0], dp = -ak[0], rp = 0.0;
+    if constexpr (!kY) {
+        // the axial terms of every row, ahead of the elimination: v is then done with
+        R = fma(-bk[0], dvp, R);
+        rp = ak[0] * dvp;
+#pragma unroll
+        for (int k = 1; k < kChunk; ++k) {
+            if (k < len) {
+                const double dv = vk[k - 1] - vk[k];
+                if (k == 1) R = fma(ak[k], dv, R);
+                else rk[k - 1] = fma(ak[k], dv, rk[k - 1]);
+                rk[k] = fma(-bk[k], dv, rk[k]);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 1; k < kChunk; ++k) {
+        if (k < len) {
+            const double a1 = ak[k], b1 = bk[k];
+            const double r = rcp_nr(D - a1);
+            const double w = a1 * r, u = R * r, f = F * r;
+            dp = fma(-E, f, dp);
+            rp = fma(-E, u, rp);
+            E = -(E * w);
+            F = -(b1 * f);
+            D = fma(-b1, w, dk[k] - b1);
+            R = fma(-b1, u, rk[k]);
+            rk[k - 1] = u;
+            dk[k - 1] = w;
+            bk[k - 1] = f;
+        }
+    }
+    if (act) {
+        double* o = rec + q.slot;
+        o[SF_D * nt] = D;
+        o[SF_R * nt] = R;
+        o[SF_E * nt] = E;
+        o[SF_F * nt] = F;
+        o[SF_DP * nt] = dp;
+        o[SF_RP * nt] = rp;
+    }
+    __syncthreads();
+    // the tree of tails, on the first wavefront: children before parents, then back.  A
+    // level waits on its children's (its parent's) terms alone: the rest of its records was
+    // requested a level earlier, and level bounds come from the lanes' registers.
+    if (t < kWave) {
+        const int nlev = __builtin_amdgcn_readfirstlane(lev[0]);
+        const bool few = nlev < kWave;
+        const int mine = few ? lev[1 + (t < nlev ? t : nlev)] : 0;
+        auto bound = [&](int l) {
+            return few ? __builtin_amdgcn_readlane(mine, l) : __builtin_amdgcn_readfirstlane(lev[1 + l]);
+        };
+        auto load_tail = [&](int s) {
+            const double* o = rec + s;
+            return SplitTail{o[SF_D * nt], o[SF_R * nt], o[SF_E * nt], o[SF_F * nt], o[SF_DP * nt], o[SF_RP * nt], kids[s]};
+        };
+        auto eliminate = [&](SplitTail c, int s) {
+            const int c0 = c.kids & 0xFFFF, cn = c.kids >> 16;
+            if (cn > 0) {                       // in child order, the first two requested together
+                const int c1 = cn > 1 ? c0 + 1 : c0;
+                const double d0 = rec[SF_DP * nt + c0], r0 = rec[SF_RP * nt + c0];
+                const double d1 = rec[SF_DP * nt + c1], r1 = rec[SF_RP * nt + c1];
+                c.D += d0;
+                c.R += r0;
+                if (cn > 1) {
+                    c.D += d1;
+                    c.R += r1;
+                    for (int k = c0 + 2; k < c0 + cn; ++k) {
+                        c.D += rec[SF_DP * nt + k];
+                        c.R += rec[SF_RP * nt + k];
+                    }
+                }
+            }
+            const double r = rcp_nr(c.D);
+            const double u = c.R * r, f = c.F * r;
+            double* o = rec + s;
+            o[SF_DP * nt] = fma(-c.E, f, c.dp);
+            o[SF_RP * nt] = fma(-c.E, u, c.rp);
+            o[SF_R * nt] = u;
+            o[SF_F * nt] = f;
+        };
+        int s1 = bound(nlev), s0 = bound(nlev - 1);
+        SplitTail nx = load_tail(s0 + t < s1 ? s0 + t : s0);
+        for (int l = nlev - 1; l >= 0; --l) {
+            const SplitTail c = nx;
+            const int n0 = l > 0 ? bound(l - 1) : 0;
+            if (l > 0) nx = load_tail(n0 + t < s0 ? n0 + t : n0);
+            if (s0 + t < s1) eliminate(c, s0 + t);
+            for (int s = s0 + kWave + t; s < s1; s += kWave) eliminate(load_tail(s), s);
+            round_boundary();
+            s1 = s0;
+            s0 = n0;
+        }
+        auto substitute = [&](int p, double u, double f, int s) { xt[s] = p == kNone ? u : fma(-f, xt[p], u); };
+        s0 = bound(0);
+        s1 = bound(1);
+        int s = s0 + t < s1 ? s0 + t : s0;
+        int np = par[s];
+        double nu = rec[SF_R * nt + s], nf = rec[SF_F * nt + s];
+        for (int l = 0; l < nlev; ++l) {
+            const int p = np;
+            const double u = nu, f = nf;
+            const int n1 = l + 1 < nlev ? bound(l + 2) : s1;
+            if (l + 1 < nlev) {
+                s = s1 + t < n1 ? s1 + t : s1;
+                np = par[s];
+                nu = rec[SF_R * nt + s];
+                nf = rec[SF_F * nt + s];
+            }
+            if (s0 + t < s1) substitute(p, u, f, s0 + t);
+            for (int k = s0 + kWave + t; k < s1; k += kWave)
+                substitute(par[k], rec[SF_R * nt + k], rec[SF_F * nt + k], k);
+            round_boundary();
+            s0 = s1;
+            s1 = n1;
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    const double xp = root ? 0.0 : xt[q.parent];
+    double x = xt[q.slot];
+#pragma unroll
+    for (int k = kChunk - 1; k >= 0; --k) {
+        if (k < len) {
+            if (k < len - 1) x = fma(-dk[k], x, fma(-bk[k], xp, rk[k]));
+            const int i = at(k);
+            // the old voltage again: kept since the load, it would cost 32 registers
+            const double vo = kX || !kY ? S.v[i] : 0.0;
+            if constexpr (kX != 0) S.vold[i] = vo;
+            S.v[i] = kY ? x : vo + x;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // events
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int delivery_step(const double* ttab, int k, int kmax, double T, double half_dt) {
@@ -1891,6 +2123,22 @@ void launch_solve(const SolveArgs& a, int max_chunks, hipStream_t s) {
     else
         hipLaunchKernelGGL(k_solve<0>, grid, block, lds, s, b, b.rounds, reinterpret_cast<const uint2*>(b.desc),
                            max_chunks);
+}
+
+void launch_solve_split(const SplitArgs& a, hipStream_t s) {
+    if (a.npack <= 0) return;
+    const size_t lds = split_lds_bytes(a.threads, a.lev_stride);
+    const dim3 grid(a.npack), block(a.threads);
+    auto go = [&](auto x, auto y) {
+        constexpr int kX = decltype(x)::value, kY = decltype(y)::value;
+        if (a.threads <= 512) hipLaunchKernelGGL((k_solve_split<kX, kY, 512>), grid, block, lds, s, a);
+        else hipLaunchKernelGGL((k_solve_split<kX, kY, kSplitMaxChunks>), grid, block, lds, s, a);
+    };
+    using std::integral_constant;
+    if (a.store_vold && a.yform) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else if (a.store_vold) go(integral_constant<int, 1>{}, integral_constant<int, 0>{});
+    else if (a.yform) go(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+    else go(integral_constant<int, 0>{}, integral_constant<int, 0>{});
 }
 
 // Streaming ceiling of the node kernel's access mix: each thread reads R fp64 columns

@@ -336,6 +336,38 @@ struct hx_sim {
     bool solve_voltage_allowed = true;   // the solve may take rhs + d v and yield v_new itself
     bool solve_voltage = false;          // in use: every d and rhs term of a step is the node kernel's
     int pass_yform = 0;                  // the node pass being launched stores rhs + d v
+    // Solve by substructuring (k_solve_split): in use when no cell has more than
+    // kSplitMaxChunks chunks and the model no more than kSplitMaxTotal.  It leaves the assembled matrix in d and rhs; the pivots and
+    // the solution go there when something reads them (make_dx): after every solve once a
+    // handle, monitor or transfer names d or rhs (need_dx), else from the call's last step
+    // (dx_pending, with its form in dx_yform and its old voltages in d_vold).
+    bool solve_split_allowed = true;
+    bool solve_split = false;
+    bool need_dx = false, dx_pending = false;
+    int dx_yform = 0;
+    double* d_vold = nullptr;
+    std::vector<SplitDesc> split_descs;
+    std::vector<int> split_levels, unit_pack_begin;
+    int split_threads = 0, split_lev_stride = 0;
+    SplitDesc* d_split_desc = nullptr;
+    int* d_split_levels = nullptr;
+    // A taped run in the voltage form keeps the rounds: its gradients are sums of terms that
+    // cancel, and carry the rounding of the solve 1000 times enlarged (12 pyramidal cells,
+    // 100 steps, against 64 bits: 3.7e-11 with the rounds, 5.6e-11 without).
+    bool use_split() const { return solve_split && !(tape_on && solve_voltage); }
+    void build_packs();
+    SolveArgs solve_args(int unit0, int unit1, bool store) const;
+    SplitArgs split_args(int unit0, int unit1) const;
+    void issue_solve(int unit0, int unit1, hipStream_t s);
+    bool reads_dx(const Ref& r) const {
+        return d_d && ((r.dev >= d_d && r.dev < d_d + nnode) || (r.dev >= d_rhs && r.dev < d_rhs + nnode));
+    }
+    void note_dx_reader(const Ref& r) {
+        if (!reads_dx(r)) return;
+        make_dx();
+        need_dx = true;
+    }
+    void make_dx();
     int res_nodes = 0;                   // in use (set at load): nodes of the largest unit, 0: streamed
     // the solver's tree (user node indices) and its coupling coefficients
     std::vector<int> solve_parent;
@@ -446,7 +478,10 @@ struct hx_sim {
     hipEvent_t ev_stagger = nullptr;     // group g's first node pass of a run, awaited by group g+1
     bool stagger_next = false;           // the next grouped step starts the groups half a step apart
     int stagger_groups = 1;              // 0: all groups start together
-    int group_turns = 1;                 // hx_set_group_turns: the groups' node passes take turns
+    // hx_set_group_turns: the groups' node passes take turns.  By default (-1) not beside
+    // the solve by substructuring, whose models are bound by the host's launches and waits:
+    // 1500 500-node cells 17.5 -> 13.4 ms for 200 steps, 21 pyramidal cells 12.6 -> 9.6 ms.
+    int group_turns = -1;
     bool turns_prev = false;             // a grouped step of this run was issued (its passes are recorded)
     // time table
     std::vector<double> ttab;
@@ -945,6 +980,7 @@ void hx_sim::build_layout() {
         U = std::max(1, U / 2);
     }
     unit_cells = U;
+    build_packs();
 
     // mechanism instance order: by solver-order node (stable); artificial cells
     // sit on no node and keep their own order
@@ -1007,6 +1043,105 @@ void hx_sim::build_layout() {
 }
 
 // the density mechanisms in the order of their kernels when they are not fused
+// The packs of k_solve_split: each unit's cells in order, as many to a pack as fit
+// kSplitPackChunks (one at least).  A unit's chunk slots are breadth-first over all its
+// cells, so the slots of a few of them in the same order are breadth-first too.
+void hx_sim::build_packs() {
+    split_descs.clear();
+    split_levels.clear();
+    unit_pack_begin.assign(nunit + 1, 0);
+    split_threads = split_lev_stride = 0;
+    solve_split = false;
+    struct Pack {
+        std::vector<SplitDesc> desc;     // by thread
+        std::vector<int> lev;            // first slot of each level, then the end
+    };
+    std::vector<Pack> packs;
+    size_t max_lev = 0;
+    int max_chunks = 0, max_nodes = 0;
+    for (int u = 0; u < nunit; ++u) {
+        unit_pack_begin[u] = static_cast<int>(packs.size());
+        const int nc = unit_desc_begin[u + 1] - unit_desc_begin[u];
+        // by slot: the chunk's descriptor, head and round, its cell (of the unit) and level
+        std::vector<const ChunkDesc*> cd(nc, nullptr);
+        std::vector<int> base(nc), rnd(nc), cell(nc), level(nc), order(nc);
+        int pos = 0;
+        for (int r = unit_round_begin[u]; r < unit_round_begin[u + 1]; ++r)
+            for (int l = 0; l < rounds[r].desc_count; ++l, ++pos) {
+                const ChunkDesc& c = descs[unit_desc_begin[u] + rounds[r].desc_begin + l];
+                cd[c.slot] = &c;
+                base[c.slot] = unit_node_begin[u] + rounds[r].node_base + l;
+                rnd[c.slot] = r;
+                order[pos] = c.slot;
+            }
+        std::vector<int> chunks_of, nodes_of;      // per cell of the unit
+        for (int q = 0; q < nc; ++q) {
+            if (cd[q]->parent_slot == kNone) {
+                cell[q] = static_cast<int>(chunks_of.size());
+                level[q] = 0;
+                chunks_of.push_back(1);
+                nodes_of.push_back(0);
+            } else {
+                cell[q] = cell[cd[q]->parent_slot];
+                level[q] = level[cd[q]->parent_slot] + 1;
+                ++chunks_of[cell[q]];
+            }
+            nodes_of[cell[q]] += cd[q]->len;
+            max_nodes = std::max(max_nodes, nodes_of[cell[q]]);
+        }
+        std::vector<int> pack_of(chunks_of.size());
+        int fill = 0;
+        for (size_t c = 0; c < chunks_of.size(); ++c) {
+            if (chunks_of[c] > kSplitMaxChunks) return;
+            if (c == 0 || fill + chunks_of[c] > kSplitPackChunks) {
+                packs.emplace_back();
+                fill = 0;
+            }
+            fill += chunks_of[c];
+            pack_of[c] = static_cast<int>(packs.size()) - 1;
+            max_chunks = std::max(max_chunks, fill);
+        }
+        std::vector<int> slot(nc), used(packs.size() - unit_pack_begin[u], 0);
+        for (int q = 0; q < nc; ++q) {
+            Pack& p = packs[pack_of[cell[q]]];
+            slot[q] = used[pack_of[cell[q]] - unit_pack_begin[u]]++;
+            if (level[q] == static_cast<int>(p.lev.size())) p.lev.push_back(slot[q]);
+        }
+        for (size_t i = 0; i < used.size(); ++i) {
+            Pack& p = packs[unit_pack_begin[u] + i];
+            p.lev.push_back(used[i]);
+            max_lev = std::max(max_lev, p.lev.size());
+        }
+        for (int q : order) {
+            SplitDesc d{};
+            d.base = base[q];
+            d.round = rnd[q];
+            d.slot = static_cast<uint16_t>(slot[q]);
+            d.parent = cd[q]->parent_slot == kNone ? kNone : static_cast<uint16_t>(slot[cd[q]->parent_slot]);
+            d.child_begin = cd[q]->child_count ? static_cast<uint16_t>(slot[cd[q]->child_begin]) : 0;
+            d.len = cd[q]->len;
+            d.child_count = cd[q]->child_count;
+            packs[pack_of[cell[q]]].desc.push_back(d);
+        }
+    }
+    unit_pack_begin[nunit] = static_cast<int>(packs.size());
+    split_threads = (max_chunks + kWave - 1) / kWave * kWave;
+    split_lev_stride = static_cast<int>(max_lev) + 1;
+    for (const Pack& p : packs) {
+        for (int i = 0; i < split_threads; ++i) {
+            SplitDesc d = p.desc[0];         // a thread past the pack's chunks reads a head and writes nothing
+            d.slot = d.parent = kNone;
+            split_descs.push_back(i < static_cast<int>(p.desc.size()) ? p.desc[i] : d);
+        }
+        split_levels.push_back(static_cast<int>(p.lev.size()) - 1);
+        for (int i = 0; i + 1 < split_lev_stride; ++i)
+            split_levels.push_back(i < static_cast<int>(p.lev.size()) ? p.lev[i] : p.lev.back());
+    }
+    const bool resident_cells = static_cast<size_t>(max_nodes) * kStageArrays * sizeof(double) <= kResUnitBudget;
+    solve_split = solve_split_allowed && !packs.empty() &&
+                  static_cast<long long>(descs.size()) <= (resident_cells ? 1 : 2) * kSplitMaxTotal;
+}
+
 static const int kSparseOrder[] = {M_PAS, M_NA_ION, M_K_ION, M_HH, M_CA_ION, M_CADYN, M_CAHVA, M_HDLA};
 
 // Fusing the state update of step k-1 into the current pass of step k is exact
@@ -1083,6 +1218,12 @@ void hx_sim::upload() {
     d_unit_round_begin = dupload(owned, unit_round_begin);
     d_rounds = dupload(owned, rounds);
     d_desc = dupload(owned, descs);
+    need_dx = dx_pending = false;
+    if (solve_split) {
+        d_split_desc = dupload(owned, split_descs);
+        d_split_levels = dupload(owned, split_levels);
+        d_vold = dalloc<double>(owned, nnode);
+    }
     {
         int dev = 0;
         hipDeviceProp_t prop;
@@ -2402,6 +2543,7 @@ void hx_sim::mirror_ab(const Ref& r, double value) {
         return;
     }
     if (!r.ab || r.node < 0) return;
+    make_dx();                         // with the coefficients of its step
     const int u = r.node;
     (r.ab == 1 ? a : b)[u] = value;
     const int p = parent[u];
@@ -2423,6 +2565,7 @@ void hx_sim::mirror_ab(const Ref& r, double value) {
 // A sampled assigned variable (klass 1) or point-process variable is only
 // valid at the reference's record point under the split schedule.
 void hx_sim::require_sample_point(const Ref& r) {
+    note_dx_reader(r);
     if ((r.klass == 1 || r.point) && !need_split_for_monitor) {
         need_split_for_monitor = true;
         write_assigned = write_assigned || r.klass == 1;
@@ -2502,6 +2645,77 @@ void hx_sim::upload_gap_ptrs() {
     }
 }
 
+// The tree solve of units [unit0, unit1) over the stepping arrays.
+SolveArgs hx_sim::solve_args(int unit0, int unit1, bool store) const {
+    SolveArgs S{};
+    S.waves = solve_waves;
+    S.nunit = unit1 - unit0;
+    S.unit_node_begin = d_unit_node_begin + unit0;
+    S.unit_desc_begin = d_unit_desc_begin + unit0;
+    S.unit_round_begin = d_unit_round_begin + unit0;
+    S.rounds = d_rounds;
+    S.desc = d_desc;
+    S.v = d_v;
+    S.d = d_d;
+    S.rhs = d_rhs;
+    S.w = d_w;
+    S.a = d_sa;
+    S.b = d_sb;
+    S.store_dx = store ? 1 : 0;
+    S.res_nodes = res_nodes;
+    S.res_rounds = max_rounds;
+    S.yform = solve_voltage ? 1 : 0;
+    return S;
+}
+
+SplitArgs hx_sim::split_args(int unit0, int unit1) const {
+    SplitArgs P{};
+    const int p0 = unit_pack_begin[unit0];
+    P.npack = unit_pack_begin[unit1] - p0;
+    P.threads = split_threads;
+    P.lev_stride = split_lev_stride;
+    P.desc = d_split_desc + static_cast<size_t>(p0) * split_threads;
+    P.levels = d_split_levels + static_cast<size_t>(p0) * split_lev_stride;
+    P.rounds = d_rounds;
+    P.v = d_v;
+    P.d = d_d;
+    P.rhs = d_rhs;
+    P.a = d_sa;
+    P.b = d_sb;
+    P.vold = d_vold;
+    P.store_vold = final_step || need_dx ? 1 : 0;
+    P.yform = solve_voltage ? 1 : 0;
+    return P;
+}
+
+void hx_sim::issue_solve(int unit0, int unit1, hipStream_t s) {
+    if (!use_split()) {
+        launch_solve(solve_args(unit0, unit1, store_dx()), max_slots, s);
+        return;
+    }
+    launch_solve_split(split_args(unit0, unit1), s);
+    if (need_dx) {
+        SolveArgs S = solve_args(unit0, unit1, true);
+        S.v = d_vold;
+        launch_solve(S, max_slots, s);
+    } else if (final_step) {
+        dx_pending = true;
+        dx_yform = solve_voltage ? 1 : 0;
+    }
+}
+
+// The pivots and the solution of the last step's solve, from the matrix and the voltages it
+// used (any pending state update and outputs pass come first: HX_SETTLE at the entry point).
+void hx_sim::make_dx() {
+    if (!dx_pending) return;
+    dx_pending = false;
+    SolveArgs S = solve_args(0, nunit, true);
+    S.v = d_vold;
+    S.yform = dx_yform;
+    launch_solve(S, max_slots, stream);
+    HXC(hipStreamSynchronize(stream));
+}
+
 bool hx_sim::want_multi_stream() const {
     return group_streams_allowed && groups.size() > 1 && fused && vecplay.empty() && !tape_on && dg_src.empty() &&
            !(learn && learn->capturing()) && (mon_ref.empty() || mon_all_v);
@@ -2535,7 +2749,7 @@ void hx_sim::step_once_groups() {
     // stream) is dispatched before the next group's node pass, which otherwise fills
     // every CU first and leaves the solve's workgroups waiting for room.  The ordering
     // is through events only: results are unchanged.
-    const bool turns = group_turns != 0;
+    const bool turns = group_turns < 0 ? !solve_split : group_turns != 0;
     const bool stagger = stagger_next && !turns;
     stagger_next = false;
     const int G = static_cast<int>(groups.size());
@@ -2577,26 +2791,8 @@ void hx_sim::step_once_groups() {
             if (stagger && g + 1 < G) HXC(hipEventRecord(ev_stagger, s));
             record();
         }
-        SolveArgs S{};
-        S.waves = solve_waves;
-        S.nunit = cg.unit1 - cg.unit0;
-        S.unit_node_begin = d_unit_node_begin + cg.unit0;
-        S.unit_desc_begin = d_unit_desc_begin + cg.unit0;
-        S.unit_round_begin = d_unit_round_begin + cg.unit0;
-        S.rounds = d_rounds;
-        S.desc = d_desc;
-        S.v = d_v;
-        S.d = d_d;
-        S.rhs = d_rhs;
-        S.w = d_w;
-        S.a = d_sa;
-        S.b = d_sb;
-        S.store_dx = store_dx() ? 1 : 0;
-        S.res_nodes = res_nodes;
-        S.res_rounds = max_rounds;
-        S.yform = solve_voltage ? 1 : 0;
         tbegin(T_SOLVE, s);
-        launch_solve(S, max_slots, s);
+        issue_solve(cg.unit0, cg.unit1, s);
         tend(T_SOLVE, s);
         // the group's detection of the next step and its synapses' decay, one launch
         tbegin(T_SPIKE, s);
@@ -2658,26 +2854,8 @@ void hx_sim::step_once() {
     }
     launch_point_currents(tmid);
     launch_plugin_currents(tmid);
-    SolveArgs S{};
-    S.waves = solve_waves;
-    S.nunit = nunit;
-    S.unit_node_begin = d_unit_node_begin;
-    S.unit_desc_begin = d_unit_desc_begin;
-    S.unit_round_begin = d_unit_round_begin;
-    S.rounds = d_rounds;
-    S.desc = d_desc;
-    S.v = d_v;
-    S.d = d_d;
-    S.rhs = d_rhs;
-    S.w = d_w;
-    S.a = d_sa;
-    S.b = d_sb;
-    S.store_dx = store_dx() ? 1 : 0;
-    S.res_nodes = res_nodes;
-    S.res_rounds = max_rounds;
-    S.yform = solve_voltage ? 1 : 0;
     tbegin(T_SOLVE);
-    launch_solve(S, max_slots, stream);
+    issue_solve(0, nunit, stream);
     tend(T_SOLVE);
     // gap transfers, detection of the next step (spike_deliver detects on v_{k}), VecPlay
     // at the step's end and the synapses' decay: one launch when VecPlay writes only IClamp
@@ -2791,7 +2969,7 @@ void hx_sim::launch_outputs_pass() {
     StepArgs A = step_args(t - 0.5 * dt, 0, 1);
     final_step = f;
     lazy_outputs_run = l;
-    A.v = d_w;
+    A.v = solve_split ? d_vold : d_w;
     A.d = d_w;
     A.rhs = d_w;
     A.fold_mask = 0;
@@ -2942,6 +3120,7 @@ int hx_sim::run_steps(int nstep) {
     // reference's last step.
     final_step = false;
     outputs_pending = false;           // this call's last step makes new ones
+    if (nstep > 0) dx_pending = false;
     lazy_outputs_run = lazy_outputs_ok();
     // cell groups on their own streams: they start after everything already on
     // the library stream, and the library stream waits for all of them
@@ -3060,6 +3239,7 @@ void hx_sim::finitialize(double v_init) {
     state_pending = false;
     pending_sampled = false;
     outputs_pending = false;
+    dx_pending = false;                // the pass below stores a new d and rhs
     lazy_outputs_run = false;
     cadyn_done = false;
     pass_cadyn_skip = pass_cadyn_after = 0;
@@ -3521,6 +3701,7 @@ int hx_load_model(hx_sim* sim) {
         if (!r.dev) return sim->fail("monitor %s.%s[%d] not found", sim->mon_name[i].first.c_str(),
                                      sim->mon_name[i].second.c_str(), sim->mon_idx[i]);
         sim->mon_ref[i] = r;
+        sim->note_dx_reader(r);
         if (r.klass == 1 || r.point) {
             // assigned outputs are sampled where the reference records them: split passes
             sim->need_split_for_monitor = true;
@@ -3612,6 +3793,8 @@ int hx_add_gap_target(hx_sim* sim, int sid, const char* mech, const char* var, i
     const Ref src = sim->resolve(it->second.mech, it->second.var, it->second.idx);
     const Ref dst = sim->resolve(mech, var, idx);
     if (!src.dev || !dst.dev) return sim->fail("Failed to resolve variable pointers");
+    sim->note_dx_reader(src);
+    sim->note_dx_reader(dst);
     it->second.targets.emplace_back(mech, var, idx);
     sim->dg_src.push_back(src.dev);
     sim->dg_dst.push_back(dst.dev);
@@ -3790,6 +3973,7 @@ int hx_get_variable_handle(hx_sim* sim, const char* mech, const char* var, int i
     Ref r = sim->resolve(mech ? mech : "", var ? var : "", idx);
     if (!r.dev) return sim->fail("variable %s.%s[%d] not found", mech, var, idx);
     if (r.klass == 1) sim->write_assigned = true;
+    sim->note_dx_reader(r);
     sim->handles.push_back(r);
     return static_cast<int>(sim->handles.size()) - 1;
     API_END
@@ -3846,6 +4030,7 @@ int hx_get_variable_value(hx_sim* sim, const char* mech, const char* var, int id
     API_BEGIN
     Ref r = sim->resolve(mech ? mech : "", var ? var : "", idx);
     if (!r.dev) return sim->fail("variable %s.%s[%d] not found", mech, var, idx);
+    if (sim->reads_dx(r)) sim->make_dx();
     HXC(hipStreamSynchronize(sim->stream));
     HXC(hipMemcpy(out, r.dev, sizeof(double), hipMemcpyDeviceToHost));
     return 0;
@@ -3858,6 +4043,7 @@ int hx_set_variable_value(hx_sim* sim, double value, const char* mech, const cha
     API_BEGIN
     Ref r = sim->resolve(mech ? mech : "", var ? var : "", idx);
     if (!r.dev) return sim->fail("variable %s.%s[%d] not found", mech, var, idx);
+    if (sim->reads_dx(r)) sim->make_dx();
     HXC(hipStreamSynchronize(sim->stream));
     HXC(hipMemcpy(r.dev, &value, sizeof(double), hipMemcpyHostToDevice));
     sim->mirror_ab(r, value);
@@ -3875,8 +4061,10 @@ int hx_get_array(hx_sim* sim, const char* mech, const char* var, double* out, in
         double* src = nullptr;
         if (mn == "capacitance") src = vn == "cm" ? sim->d_cm : nullptr;
         else if (vn == "v") src = sim->d_v;
-        else if (vn == "d") src = sim->d_d;
-        else if (vn == "rhs") src = sim->d_rhs;
+        else if (vn == "d" || vn == "rhs") {
+            sim->make_dx();
+            src = vn == "d" ? sim->d_d : sim->d_rhs;
+        }
         else if (vn == "a") src = sim->d_a;
         else if (vn == "b") src = sim->d_b;
         else if (vn == "area") src = sim->d_area;
@@ -4123,6 +4311,13 @@ int hx_set_solve_resident(hx_sim* sim, int enable) {
     HX_SETTLE(sim);
     if (sim->loaded) return sim->fail("choose the tree solve's kernel before hx_load_model");
     sim->solve_resident_allowed = enable != 0;
+    return 0;
+}
+
+int hx_set_solve_split(hx_sim* sim, int enable) {
+    HX_SETTLE(sim);
+    if (sim->loaded) return sim->fail("choose the tree solve's kernel before hx_load_model");
+    sim->solve_split_allowed = enable != 0;
     return 0;
 }
 
@@ -4427,6 +4622,7 @@ long long hx_get_info(hx_sim* sim, const char* key) {
     if (k == "solve_unit_cells") return sim->unit_cells;
     if (k == "solve_waves") return sim->solve_waves;
     if (k == "solve_resident") return sim->res_nodes > 0 ? 1 : 0;
+    if (k == "solve_split") return sim->solve_split ? 1 : 0;
     if (k == "solve_voltage") return sim->solve_voltage ? 1 : 0;
     if (k == "nchunk_total") return static_cast<long long>(sim->descs.size());
     if (k == "event_slots") return sim->groups.empty() ? 0 : sim->groups[0].ring.nslot;
@@ -4751,25 +4947,29 @@ int hx_adjoint(hx_sim* sim, int nloss, const int* loss_nodes, const double* targ
     A.loss_scale = scale;
     sim->adj_fuse_bits = A.fuse_state | (A.fuse_cond << 8) | (A.fuse_param << 16) |
                          (static_cast<unsigned>(A.fold_syn) << 24) | ((d_lmap ? 1u : 0u) << 25);
-    SolveArgs S{};
-    S.waves = sim->solve_waves;
-    S.nunit = sim->nunit;
-    S.unit_node_begin = sim->d_unit_node_begin;
-    S.unit_desc_begin = sim->d_unit_desc_begin;
-    S.unit_round_begin = sim->d_unit_round_begin;
-    S.rounds = sim->d_rounds;
-    S.desc = sim->d_desc;
+    // M^T: the coefficients trade places.  D and x are not needed, and the transposed
+    // system's unknown starts at 0, so the solve reads no v and the new v it writes is the
+    // solution itself.
+    SolveArgs S = sim->solve_args(0, sim->nunit, false);
     S.v = sim->d_vT;
     S.d = sim->d_dT;
     S.rhs = sim->d_rhsT;
     S.w = sim->d_wT;
-    S.a = sim->d_sb;      // M^T: the coefficients trade places
+    S.a = sim->d_sb;
     S.b = sim->d_sa;
-    S.store_dx = 0;       // D and x are not needed
-    S.yform = 1;          // the transposed system's unknown starts at 0: the solve reads no v,
-                          // and the new v it writes is the solution itself
-    S.res_nodes = sim->res_nodes;
-    S.res_rounds = sim->max_rounds;
+    S.yform = 1;
+    SplitArgs P{};
+    const bool split = sim->use_split();
+    if (split) {
+        P = sim->split_args(0, sim->nunit);
+        P.v = S.v;
+        P.d = S.d;
+        P.rhs = S.rhs;
+        P.a = S.a;
+        P.b = S.b;
+        P.yform = 1;
+        P.store_vold = 0;
+    }
     double* lv = sim->d_lv;
     double* lv2 = sim->d_lv2;
     const size_t row = static_cast<size_t>(N);
@@ -4791,7 +4991,8 @@ int hx_adjoint(hx_sim* sim, int nloss, const int* loss_nodes, const double* targ
         A.loss_v = (d_lmap && n >= 1) ? sim->d_tape_v + (n - 1) * row : nullptr;
         A.loss_tgt = n >= 1 ? d_tgt + static_cast<size_t>(n - 1) * nloss : nullptr;
         launch_adj_before_solve(A, st);
-        launch_solve(S, sim->max_slots, st);
+        if (split) launch_solve_split(P, st);
+        else launch_solve(S, sim->max_slots, st);
         launch_adj_after_solve(A, st);
         if (n >= 1 && !d_lmap)
             launch_adj_loss(sim->d_tape_v + (n - 1) * row, d_un, d_ubeg, d_uidx, nun,

@@ -142,6 +142,7 @@ SIGNATURES = {
     "hx_set_solve_unit_cells": (C.c_int, [_P, C.c_int]),
     "hx_set_solve_waves": (C.c_int, [_P, C.c_int]),
     "hx_set_solve_resident": (C.c_int, [_P, C.c_int]),
+    "hx_set_solve_split": (C.c_int, [_P, C.c_int]),
     "hx_set_solve_voltage": (C.c_int, [_P, C.c_int]),
     "hx_output_spikes": (C.c_int, [_P, C.c_char_p]),
     "hx_set_spike_output_enabled": (C.c_int, [_P, C.c_int]),
@@ -1087,6 +1088,11 @@ class Sim:
         """Hold each solve unit whole in LDS when it fits (the default) or always stream its
         rounds from HBM.  Call before loading the model; the same bits either way."""
         self._chk(lib().hx_set_solve_resident(self._h, int(bool(enable))), "set_solve_resident")
+
+    def set_solve_split(self, enable: bool) -> None:
+        """Solve by substructuring where every cell allows it (the default) or always round by
+        round.  Call before loading the model; the two agree to rounding."""
+        self._chk(lib().hx_set_solve_split(self._h, int(bool(enable))), "set_solve_split")
 
     def set_solve_voltage(self, enable: bool) -> None:
         """Let a model whose node kernel makes every term of d and rhs solve for the new

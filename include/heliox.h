@@ -320,6 +320,14 @@ int hx_set_solve_waves(hx_sim* sim, int waves);
  * a larger unit: the rounds are streamed through LDS from HBM.  The same bits either way;
  * hx_get_info("solve_resident") reports the choice.  Call before hx_load_model. */
 int hx_set_solve_resident(hx_sim* sim, int enable);
+/* Tree solve by substructuring (no counterpart in the reference): enable = 1 (default) lets
+ * every unbranched run of up to 16 nodes eliminate its interior at once, one thread each,
+ * and solves the tree of the runs' tails level by level, where no cell has more than 768
+ * such runs and the model no more than 196608 (393216 with cells above 1024 nodes); 0
+ * solves round by round (hx_set_solve_resident), which also yields d and rhs after a step
+ * in either case.  The two agree to rounding.  hx_get_info("solve_split") reports the
+ * choice.  Call before hx_load_model. */
+int hx_set_solve_split(hx_sim* sim, int enable);
 /* Tree solve unknown (no counterpart in the reference): enable = 1 (default) lets a model
  * whose node kernel makes every term of d and rhs (no density mechanism on its own kernel,
  * no IClamp or HalfGap instance, no plugin) store rhs + d v, so that the solve yields the

@@ -1,0 +1,117 @@
+"""The tree solve by substructuring (k_solve_split) against the round-by-round solve and the
+oracle, at the sizes where it could go wrong: cells of a single node, of one chunk and one
+more, packs of several cells, a level wider than a wavefront, more chunks than 512 threads
+and more than the kernel takes; with the voltage and with the change as the unknown; the
+pivots and the solution read after a step, through a handle, and after a coefficient changed."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle
+from heliox_amd import Sim, build_config
+from heliox_amd.spec import MechSpec, ModelSpec
+from parity_util import V_TOL
+
+pytestmark = pytest.mark.gpu
+
+# Rounding alone separates the two orders of elimination: a step leaves a few ulp of v
+# (1.4e-14 mV at 65 mV) times the matrix' condition (couplings of at most 4 a node over the
+# capacitive 0.04: 100), and the cells are passive, so 40 steps stay below 1e-10 mV.
+TOL = 1e-10
+
+
+def chain(n):
+    return [-1] + list(range(n - 1))
+
+
+def star(n):
+    return [-1] + [0] * (n - 1)
+
+
+def bushy(n):
+    rng = np.random.default_rng(n)
+    return [-1] + [int(rng.integers(max(0, i - 6), i)) for i in range(1, n)]
+
+
+def passive(parents, ncell, clamp):
+    """`ncell` copies of one tree with unequal couplings, pas everywhere; `clamp` adds a current
+    injection, which leaves the change as the unknown."""
+    m, n = len(parents), len(parents) * ncell
+    node = np.empty((ncell, m), np.int64)
+    node[:, 0] = np.arange(ncell)
+    node[:, 1:] = ncell + np.arange(ncell * (m - 1)).reshape(ncell, m - 1)
+    par = np.full(n, -1, np.int32)
+    for c in range(ncell):
+        par[node[c, 1:]] = node[c, np.asarray(parents[1:], np.int64)]
+    rng = np.random.default_rng(31 * m + ncell)
+    a, b = -rng.uniform(0.05, 2.0, n), -rng.uniform(0.05, 2.0, n)
+    deg = np.bincount(par[ncell:], minlength=n) if m > 1 else np.zeros(n)
+    a[ncell:] /= np.maximum(1.0, deg[par[ncell:]])
+    a[:ncell] = b[:ncell] = 0.0
+    mechs = {"pas": MechSpec(np.arange(n, dtype=np.int32),
+                             {"g_pas": rng.uniform(1e-4, 1e-3, n), "e_pas": rng.uniform(-75.0, -60.0, n)})}
+    if clamp:
+        mechs["IClamp"] = MechSpec(np.arange(ncell, dtype=np.int32),
+                                   {"delay": np.full(ncell, 0.2), "dur": np.full(ncell, 5.0), "amp": np.full(ncell, 0.1)})
+    return ModelSpec(ncell=ncell, parent=par, a=a, b=b, area=rng.uniform(50.0, 500.0, n), cm=np.ones(n), mechs=mechs)
+
+
+def run(spec, split, tstop=1.0, groups=1, unit_cells=0, handle=None):
+    g = Sim()
+    g.set_cell_groups(groups)
+    g.set_solve_unit_cells(unit_cells)
+    g.set_solve_split(split)
+    g.load_model_from_spec(dataclasses.replace(spec, monitors=[("global", "v", c) for c in range(spec.ncell)]))
+    if handle:
+        g.get_variable_handle(*handle)
+    g.finitialize(-65.0)
+    for _ in range(2):
+        g.continue_run(tstop / 2)
+    return g
+
+
+@pytest.mark.parametrize("clamp", [False, True])
+@pytest.mark.parametrize("shape,size,ncell,takes", [
+    (chain, 1, 3, 1), (chain, 16, 5, 1), (chain, 17, 5, 1), (chain, 101, 9, 1), (star, 71, 2, 1), (bushy, 40, 30, 1),
+    (bushy, 260, 3, 1), (bushy, 1000, 2, 1), (bushy, 1600, 1, 0)])
+def test_split_solve_matches_the_rounds(gpu_lib, shape, size, ncell, takes, clamp):
+    print(f"case split {shape.__name__} {size} x {ncell} clamp={clamp}", flush=True)
+    spec = passive(shape(size), ncell, clamp)
+    s, r = run(spec, True), run(spec, False)
+    print("chunks", s.info("nchunk_total"), flush=True)
+    assert s.info("solve_split") == takes and r.info("solve_split") == 0
+    assert s.info("solve_voltage") == int(not clamp)
+    assert float(np.max(np.abs(s.traces() - r.traces()))) < TOL
+    for k in ("v", "rhs"):
+        assert float(np.max(np.abs(s.get_array("global", k) - r.get_array("global", k)))) < TOL, k
+    np.testing.assert_allclose(s.get_array("global", "d"), r.get_array("global", "d"), rtol=TOL)
+    o = oracle.OracleSim(spec, monitors=[("global", "v", c) for c in range(ncell)])
+    o.finitialize(-65.0)
+    for _ in range(2):
+        o.continue_run(0.5)
+    assert float(np.max(np.abs(o.traces() - s.traces()))) < V_TOL
+
+
+@pytest.mark.parametrize("unit_cells,groups", [(1, 1), (7, 1), (3, 2)])
+def test_packs_change_no_bit(gpu_lib, unit_cells, groups):
+    print(f"case split packs unit_cells={unit_cells} groups={groups}", flush=True)
+    spec = build_config(5, 20, 5.0)
+    base, g = run(spec, True, 5.0), run(spec, True, 5.0, groups, unit_cells)
+    assert g.info("solve_split") == 1
+    assert np.array_equal(base.traces(), g.traces())
+    assert np.array_equal(base.get_array("global", "v"), g.get_array("global", "v"))
+
+
+def test_pivots_and_solution_on_demand(gpu_lib):
+    spec = passive(bushy(60), 4, False)
+    print("case split on demand", flush=True)
+    plain, held = run(spec, True), run(spec, True, handle=("global", "rhs", 5))
+    assert np.array_equal(plain.traces(), held.traces())        # a reader of rhs changes no voltage
+    late = run(spec, True)
+    late.set_variable_value(-1.5, "global", "a", 50)            # after the step that d and rhs belong to
+    for k in ("d", "rhs"):
+        want = plain.get_array("global", k)
+        assert np.array_equal(held.get_array("global", k), want), k
+        assert np.array_equal(late.get_array("global", k), want), k
+    assert held.get_variables_by_handles([0])[0] == plain.get_variable_value("global", "rhs", 5)
