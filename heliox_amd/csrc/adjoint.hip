@@ -478,14 +478,28 @@ __global__ void k_adj_gather(const double* tape_v, long long row, const int* nod
     out[t] = tape_v[r * row + nodes[j]];
 }
 
-// Adam: one thread per tied group (optimizer.cpp:351-393, optimizer_kernels.cu:173-195)
-__global__ void k_adam(AdamArgs A) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+// Optimizer step, one wavefront per tied group (optimizer.cpp:351-393,
+// optimizer_kernels.cu:173-195).  A tied group is a cell's compartments, up to thousands of
+// entries behind pointers: one thread walked them as a serial chain of two dependent loads
+// (60 groups of 5000 and 2400 of one: 2.6 ms; 600 of 50 to 500: 0.41 ms; a wavefront each
+// 0.1 ms and less).
+// The lanes load 64 entries at a time; the sum is taken in list order, the serial walk's bits.
+__global__ void __launch_bounds__(kBlock) k_adam(AdamArgs A) {
+    const int g = (blockIdx.x * kBlock + threadIdx.x) / kWave;
+    const int lane = threadIdx.x % kWave;
     if (g >= A.ngroup) return;
     const int b0 = A.begin[g], b1 = A.begin[g + 1];
     if (b1 <= b0) return;
-    double sum = 0.0;
-    for (int k = b0; k < b1; ++k) sum += *A.grad[k];
+    auto load = [&](int k) { return k < b1 ? *A.grad[k] : 0.0; };
+    double sum = 0.0, next = load(b0 + lane);
+    for (int c = b0; c < b1; c += kWave) {
+        const double x = next;
+        next = load(c + kWave + lane);
+        const int lo = __double2loint(x), hi = __double2hiint(x);
+        const int n = b1 - c < kWave ? b1 - c : kWave;
+        for (int i = 0; i < n; ++i)
+            sum += __hiloint2double(__builtin_amdgcn_readlane(hi, i), __builtin_amdgcn_readlane(lo, i));
+    }
     const double avg = sum / static_cast<double>(b1 - b0);
     const double sg = avg * A.impedance[g] * A.inv_record_steps;
     double w;
@@ -493,18 +507,20 @@ __global__ void k_adam(AdamArgs A) {
         w = *A.w[b0] - A.lr * sg;
     } else if (A.type == 1) {
         const double vel = A.momentum * A.m[g] - A.lr * sg;
-        A.m[g] = vel;
+        if (lane == 0) A.m[g] = vel;
         w = *A.w[b0] + vel;
     } else {
         const double m = A.beta1 * A.m[g] + (1.0 - A.beta1) * sg;
         const double v = A.beta2 * A.v[g] + (1.0 - A.beta2) * sg * sg;
-        A.m[g] = m;
-        A.v[g] = v;
+        if (lane == 0) {
+            A.m[g] = m;
+            A.v[g] = v;
+        }
         const double mhat = m / (1.0 - pow(A.beta1, static_cast<double>(A.step)));
         const double vhat = v / (1.0 - pow(A.beta2, static_cast<double>(A.step)));
         w = *A.w[b0] - A.lr * mhat / (sqrt(vhat) + A.eps);
     }
-    for (int k = b0; k < b1; ++k) {
+    for (int k = b0 + lane; k < b1; k += kWave) {
         *A.w[k] = w;
         *A.grad[k] = 0.0;
     }
@@ -650,7 +666,7 @@ void launch_adj_gather(const double* tape_v, long long row, const int* nodes, in
 }
 
 void launch_adam(const AdamArgs& a, hipStream_t s) {
-    if (a.ngroup > 0) hipLaunchKernelGGL(k_adam, grid_of(a.ngroup), dim3(kBlock), 0, s, a);
+    if (a.ngroup > 0) hipLaunchKernelGGL(k_adam, grid_of(static_cast<long long>(a.ngroup) * kWave), dim3(kBlock), 0, s, a);
 }
 
 }  // namespace hx
