@@ -329,49 +329,73 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
     }
 }
 
+constexpr int kFinishMost = 16;     // elements a thread of k_rp_finish takes at once, at most
+constexpr int kFinishBlocks = 4096; // blocks of it, at most
+// Row and column of element e, kThreads after the one they hold.  A 64-bit division costs as
+// much as the rest of an element, so wide slices (N > kThreads) step instead.
+template <class I>
+__device__ __forceinline__ void next_element(I e, I N, I& row, I& col) {
+    if constexpr (sizeof(I) == 8) {
+        col += kThreads;
+        if (col >= N) {
+            col -= N;
+            ++row;
+        }
+    } else {
+        row = e / N;
+        col = e - row * N;
+    }
+}
+
 // The tick's slice from the correction's split sums, added in split order (nsplit 0: no
 // correction), kE elements per thread; the previous tick's dx on blocks of its own.  The
 // splits are read four at a time, so a thread has 4 kE loads in flight (one at a time,
-// waiting for each, the kernel took 52 us at N = 400 with 28 splits).
-template <int kE>
+// waiting for each, the kernel took 52 us at N = 400 with 28 splits).  I indexes the N x N
+// elements: unsigned, or 64 bits from about N = 65400.
+template <int kE, class I>
 __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
     __shared__ double sh[kThreads];
     if (static_cast<int>(blockIdx.x) >= A.nblock) {
         rp_dx<kThreads>(A.dx, A.O.N, blockIdx.x - A.nblock, reinterpret_cast<float*>(sh));
         return;
     }
-    const unsigned N = A.O.N, total = N * N;
-    const unsigned e0 = blockIdx.x * kE * kThreads + threadIdx.x;
+    const I N = A.O.N, total = N * N;
     const float gs = *A.O.gs;
-    float c[kE];
-    unsigned at[kE];
-#pragma unroll
-    for (int r = 0; r < kE; ++r) {
-        c[r] = 0.f;
-        at[r] = min(e0 + r * kThreads, total - 1);
-    }
-    int sp = 0;
-    for (; sp + 4 <= A.nsplit; sp += 4) {
-        float x[4][kE];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < kE; ++r) x[q][r] = A.part[static_cast<size_t>(sp + q) * total + at[r]];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < kE; ++r) c[r] += x[q][r];
-    }
-    for (; sp < A.nsplit; ++sp)
-#pragma unroll
-        for (int r = 0; r < kE; ++r) c[r] += A.part[static_cast<size_t>(sp) * total + at[r]];
     double sq = 0.0;
+    // one turn but for the largest slices, whose blocks are bounded (rp_finish_blocks)
+    for (I e0 = static_cast<I>(blockIdx.x) * kE * kThreads + threadIdx.x; e0 < total;
+         e0 += static_cast<I>(A.nblock) * kE * kThreads) {
+        float c[kE];
+        I at[kE];
 #pragma unroll
-    for (int r = 0; r < kE; ++r) {
-        if (e0 + r * kThreads >= total) break;
-        const unsigned row = at[r] / N, col = at[r] - row * N;
-        const int b = A.col_block[col];
-        A.O.out[at[r]] = rp_element(A.O, c[r], row, col, A.start[b], A.bn[b], A.O.base + A.boff[b], gs, sq);
+        for (int r = 0; r < kE; ++r) {
+            c[r] = 0.f;
+            at[r] = min(e0 + r * kThreads, total - 1);
+        }
+        int sp = 0;
+        for (; sp + 4 <= A.nsplit; sp += 4) {
+            float x[4][kE];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < kE; ++r) x[q][r] = A.part[static_cast<size_t>(sp + q) * total + at[r]];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < kE; ++r) c[r] += x[q][r];
+        }
+        for (; sp < A.nsplit; ++sp)
+#pragma unroll
+            for (int r = 0; r < kE; ++r) c[r] += A.part[static_cast<size_t>(sp) * total + at[r]];
+        I row = e0 / N, col = e0 - row * N;
+#pragma unroll
+        for (int r = 0; r < kE; ++r) {
+            if (e0 + r * kThreads >= total) break;
+            if (r > 0) next_element<I>(at[r], N, row, col);
+            const int b = A.col_block[col];
+            A.O.out[at[r]] = rp_element(A.O, c[r], row, col, A.start[b], A.bn[b], A.O.base + A.boff[b], gs, sq);
+        }
+        if constexpr (kE < kFinishMost) break;
     }
     if (A.O.sanitize) {
         const double t = block_sum<kThreads>(sq, sh);
@@ -387,19 +411,20 @@ __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
 // the same order (a launch of its own took 4 us); block 0 stores it with the rescaled
 // scales, which only later launches read.  w_tick (replay_dw_dx.cu:96-114): one wave per
 // row.  The remaining blocks form X of this tick from its slice.
-constexpr int kGather = 4;
+template <int kGather, class I>
 __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
     __shared__ double sh[kThreads];
     const int tid = threadIdx.x;
     const unsigned N = A.N;
     if (static_cast<int>(blockIdx.x) >= A.wblocks) {
-        const unsigned total = N * N;
-        const unsigned e0 = (blockIdx.x - A.wblocks) * kGather * kThreads + tid;
+        const I total = static_cast<I>(N) * N;
+        const I e0 = static_cast<I>(blockIdx.x - A.wblocks) * kGather * kThreads + tid;
+        I row = e0 / N, c = e0 - row * N;
 #pragma unroll
         for (int r = 0; r < kGather; ++r) {
-            const unsigned e = e0 + r * kThreads;
+            const I e = e0 + r * kThreads;
             if (e >= total) break;
-            const unsigned row = e / N, c = e - row * N;
+            if (r > 0) next_element<I>(e, N, row, c);
             const int p = A.pre[c], b = A.col_block[c];
             const float g = p >= 0 ? A.cur[static_cast<size_t>(row) * N + p] : 0.f;
             A.x[A.xoff[b] + static_cast<size_t>(row) * A.bnp[b] + c - A.start[b]] =
@@ -502,34 +527,49 @@ void launch_rp_corr(const ReplayCorrArgs& a, int tile_cols, hipStream_t s) {
 }
 
 // Elements per thread of k_rp_finish: one while that gives no more than about 1024 blocks
-// (every w_tick workgroup adds up the blocks' norm partials), then as many as keep it so.
+// (every w_tick workgroup adds up the blocks' norm partials), then as many as keep it so, up
+// to kFinishMost in kFinishBlocks blocks that then take turns.
 static int finish_elems(int N) {
     const long long blocks = (static_cast<long long>(N) * N + kThreads - 1) / kThreads;
-    return blocks <= 1024 ? 1 : blocks <= 4096 ? 4 : blocks <= 16384 ? 8 : 16;
+    return blocks <= 1024 ? 1 : blocks <= 4096 ? 4 : blocks <= 16384 ? 8 : kFinishMost;
 }
 
 int rp_finish_blocks(int N) {
     const long long per = static_cast<long long>(finish_elems(N)) * kThreads;
-    return static_cast<int>((static_cast<long long>(N) * N + per - 1) / per);
+    return static_cast<int>(std::min<long long>((static_cast<long long>(N) * N + per - 1) / per, kFinishBlocks));
+}
+
+// The N x N elements are indexed in 32 bits: so must be what a block's next turn starts at.
+static bool narrow_slice(int N) {
+    const long long turn = static_cast<long long>(kFinishBlocks) * kFinishMost * kThreads;
+    return static_cast<long long>(N) * N + turn < 1LL << 32;
 }
 
 void launch_rp_finish(ReplayFinishArgs a, hipStream_t s) {
     a.nblock = rp_finish_blocks(a.O.N);
     const dim3 grid(a.nblock + a.dx.n_in);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, a); };
     switch (finish_elems(a.O.N)) {
-        case 1: hipLaunchKernelGGL(k_rp_finish<1>, grid, dim3(kThreads), 0, s, a); break;
-        case 4: hipLaunchKernelGGL(k_rp_finish<4>, grid, dim3(kThreads), 0, s, a); break;
-        case 8: hipLaunchKernelGGL(k_rp_finish<8>, grid, dim3(kThreads), 0, s, a); break;
-        default: hipLaunchKernelGGL(k_rp_finish<16>, grid, dim3(kThreads), 0, s, a); break;
+        case 1: go(k_rp_finish<1, unsigned>); break;
+        case 4: go(k_rp_finish<4, unsigned>); break;
+        case 8: go(k_rp_finish<8, unsigned>); break;
+        default:
+            if (narrow_slice(a.O.N)) go(k_rp_finish<kFinishMost, unsigned>);
+            else go(k_rp_finish<kFinishMost, unsigned long long>);
     }
 }
 
 void launch_rp_tick(ReplayTickArgs a, hipStream_t s) {
-    const long long per = static_cast<long long>(kGather) * kThreads;
     a.wblocks = a.dl ? (a.N + kThreads / 64 - 1) / (kThreads / 64) : 0;
-    const long long gather = a.x ? (static_cast<long long>(a.N) * a.N + per - 1) / per : 0;
-    if (a.wblocks + gather > 0)
-        hipLaunchKernelGGL(k_rp_tick, dim3(static_cast<unsigned>(a.wblocks + gather)), dim3(kThreads), 0, s, a);
+    auto go = [&](auto kernel, int elems) {
+        const long long per = static_cast<long long>(elems) * kThreads;
+        const long long gather = a.x ? (static_cast<long long>(a.N) * a.N + per - 1) / per : 0;
+        if (a.wblocks + gather > 0)
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.wblocks + gather)), dim3(kThreads), 0, s, a);
+    };
+    // wide slices: enough elements a thread that the launch holds less than 2^32 of them
+    if (narrow_slice(a.N)) go(k_rp_tick<4, unsigned>, 4);
+    else go(k_rp_tick<16, unsigned long long>, 16);
 }
 
 void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s) {
