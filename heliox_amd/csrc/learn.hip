@@ -200,13 +200,13 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
     __shared__ __align__(16) float Bs[2][TJ][kLd];
     __shared__ double red_s[S::NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (static_cast<int>(blockIdx.x) >= A.ncorr) {            // the previous tick's dx
-        rp_dx<S::kT>(A.dx, A.O.N, blockIdx.x - A.ncorr, &As[0][0][0]);
+    int wg = static_cast<int>(blockIdx.x + blockIdx.y * gridDim.x);
+    if (wg >= A.ncorr) {                                      // the previous tick's dx
+        if (wg < A.ncorr + A.dx.n_in) rp_dx<S::kT>(A.dx, A.O.N, wg - A.ncorr, &As[0][0][0]);
         return;
     }
     // workgroups go to the eight XCDs in turn: give each XCD a run of consecutive tiles, so
     // the row tiles that share a block's taps read them from one L2
-    int wg = blockIdx.x;
     if (A.ncorr % 8 == 0) wg = (wg & 7) * (A.ncorr >> 3) + (wg >> 3);
     const int rt = wg % A.row_tiles;
     const int q = wg / A.row_tiles;
@@ -515,7 +515,11 @@ int rp_corr_splits(int N, int ntiles, int max_bnp, int tw) {
 
 template <int TJ>
 void launch_corr_tile(const ReplayCorrArgs& a, hipStream_t s) {
-    const dim3 grid(a.ncorr + a.dx.n_in), block(CorrShape<TJ>::kT);
+    // a launch holds less than 2^32 threads along x: many workgroups take rows of kCorrRow
+    // (a multiple of the XCD count, so the mapping to them stays)
+    const int total = a.ncorr + a.dx.n_in;
+    constexpr int kCorrRow = 1 << 20;
+    const dim3 grid(std::min(total, kCorrRow), (total + kCorrRow - 1) / kCorrRow), block(CorrShape<TJ>::kT);
     if (a.nsplit > 1) hipLaunchKernelGGL((k_rp_corr<TJ, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((k_rp_corr<TJ, false>), grid, block, 0, s, a);
 }

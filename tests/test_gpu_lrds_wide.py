@@ -1,5 +1,5 @@
-"""Replays whose dv/dw slice has more than 2^32 elements, and the largest indexed in 32 bits,
-against the oracle.
+"""Replays whose dv/dw slice has more than 2^32 elements, or whose correction has more
+workgroups than one row of its grid, against the oracle.
 
 All kernels are zero but those of a few blocks (the first, one in the middle, the last
 two), so nothing else ever leaves zero: the oracle runs the few blocks alone, and every
@@ -27,6 +27,7 @@ def sim(gpu_lib):
     (32, 2048, 3, 2, False, 0.5),        # N = 65539: N^2 = 2^32 + 393225
     (32, 2048, 3, 2, True, 0.5),
     (32, 2043, 31, 2, False, 0.4),       # N = 65407: the last in 32 bits
+    (2, 32769, 1, 1, True, 0.08),        # 32770 column tiles of 513 row tiles, 256 threads each
 ])
 def test_wide_replay_matches_oracle(sim, bn, nblk, last, K_len, percise, thr):
     N, ksteps = bn * nblk + last, 5
