@@ -121,10 +121,11 @@ __device__ __forceinline__ V block_sum(V x, V* sh) {
 // One element of a tick's slice from its correction sum c (replay_dw_dx.cu:227-325): base
 // term added inside the row's own block; on clip ticks non-finite entries become 0 and the
 // square goes to the norm.
+template <class Base>
 __device__ __forceinline__ float rp_element(const ReplayOut& O, float c, int row, int col, int s, int bn,
-                                            const float* base, float gs, double& sq) {
+                                            const Base& base, float gs, double& sq) {
     float v = c * O.dt;
-    if (row >= s && row < s + bn) v = base[static_cast<size_t>(row - s) * bn + col - s] * O.dt * gs + v;
+    if (row >= s && row < s + bn) v = base()[static_cast<size_t>(row - s) * bn + col - s] * O.dt * gs + v;
     if (O.sanitize) {
         if (!isfinite(v)) v = 0.f;
         sq += static_cast<double>(v) * v;
@@ -304,7 +305,8 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
     // of its wave's sub-tile
     double sq = 0.0;
     const float gs = *A.O.gs;
-    const float* base = A.O.base + A.boff[b];
+    const float* base_b = A.O.base + A.boff[b];
+    auto base = [&] { return base_b; };
     float* out = kPart ? A.part + static_cast<size_t>(sp) * N * N : A.O.out;
 #pragma unroll
     for (int n = 0; n < S::NC; ++n) {
@@ -331,26 +333,23 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
 
 constexpr int kFinishMost = 16;     // elements a thread of k_rp_finish takes at once, at most
 constexpr int kFinishBlocks = 4096; // blocks of it, at most
-// Row and column of element e, kThreads after the one they hold.  A 64-bit division costs as
-// much as the rest of an element, so wide slices (N > kThreads) step instead.
+// Row and column of the element kThreads after the one they hold.  A division costs as much
+// as the rest of an element (64 bits: more), so slices wider than kThreads step instead.
 template <class I>
-__device__ __forceinline__ void next_element(I e, I N, I& row, I& col) {
-    if constexpr (sizeof(I) == 8) {
-        col += kThreads;
-        if (col >= N) {
-            col -= N;
-            ++row;
-        }
-    } else {
-        row = e / N;
-        col = e - row * N;
+__device__ __forceinline__ void next_element(I N, I& row, I& col) {
+    col += kThreads;
+    if (col >= N) {
+        col -= N;
+        ++row;
     }
 }
 
 // The tick's slice from the correction's split sums, added in split order (nsplit 0: no
 // correction), kE elements per thread; the previous tick's dx on blocks of its own.  The
 // splits are read four at a time, so a thread has 4 kE loads in flight (one at a time,
-// waiting for each, the kernel took 52 us at N = 400 with 28 splits).  I indexes the N x N
+// waiting for each, the kernel took 52 us at N = 400 with 28 splits); so are the block
+// look-ups of a thread's columns (a division, a look-up and a store one element after the
+// other: 4.2 ms at N = 32768 without splits, now 1.4; 4.3 GB written take 0.85).  I indexes the N x N
 // elements: unsigned, or 64 bits from about N = 65400.
 template <int kE, class I>
 __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
@@ -387,14 +386,29 @@ __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
         for (; sp < A.nsplit; ++sp)
 #pragma unroll
             for (int r = 0; r < kE; ++r) c[r] += A.part[static_cast<size_t>(sp) * total + at[r]];
-        I row = e0 / N, col = e0 - row * N;
+        I row[kE], col[kE];
+        int b[kE], s[kE], bn[kE];
+        row[0] = e0 / N;
+        col[0] = e0 - row[0] * N;
 #pragma unroll
         for (int r = 0; r < kE; ++r) {
-            if (e0 + r * kThreads >= total) break;
-            if (r > 0) next_element<I>(at[r], N, row, col);
-            const int b = A.col_block[col];
-            A.O.out[at[r]] = rp_element(A.O, c[r], row, col, A.start[b], A.bn[b], A.O.base + A.boff[b], gs, sq);
+            if (r > 0) {
+                row[r] = row[r - 1];
+                col[r] = col[r - 1];
+                next_element<I>(N, row[r], col[r]);
+            }
+            b[r] = A.col_block[col[r]];
         }
+#pragma unroll
+        for (int r = 0; r < kE; ++r) {
+            s[r] = A.start[b[r]];
+            bn[r] = A.bn[b[r]];
+        }
+#pragma unroll
+        for (int r = 0; r < kE; ++r)
+            if (e0 + r * kThreads < total)
+                A.O.out[at[r]] = rp_element(A.O, c[r], row[r], col[r], s[r], bn[r],
+                                            [&] { return A.O.base + A.boff[b[r]]; }, gs, sq);
         if constexpr (kE < kFinishMost) break;
     }
     if (A.O.sanitize) {
@@ -419,12 +433,17 @@ __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
     if (static_cast<int>(blockIdx.x) >= A.wblocks) {
         const I total = static_cast<I>(N) * N;
         const I e0 = static_cast<I>(blockIdx.x - A.wblocks) * kGather * kThreads + tid;
-        I row = e0 / N, c = e0 - row * N;
+        I row = e0 / static_cast<I>(N), c = e0 - row * N;
 #pragma unroll
         for (int r = 0; r < kGather; ++r) {
             const I e = e0 + r * kThreads;
             if (e >= total) break;
-            if (r > 0) next_element<I>(e, N, row, c);
+            if constexpr (sizeof(I) == 8) {
+                if (r > 0) next_element<I>(N, row, c);
+            } else {
+                row = e / N;
+                c = e - row * N;
+            }
             const int p = A.pre[c], b = A.col_block[c];
             const float g = p >= 0 ? A.cur[static_cast<size_t>(row) * N + p] : 0.f;
             A.x[A.xoff[b] + static_cast<size_t>(row) * A.bnp[b] + c - A.start[b]] =

@@ -38,6 +38,10 @@ CASES = [
     ((16, 17), 64, 70, True, 1e6, False),
     ((70, 58), 6, 19, False, 0.05, False),
     ((40, 23), 5, 12, True, 1.0, True),
+    # more than one element a thread where the splits are summed: 4, 8 and 16
+    ((200, 199, 131), 2, 7, True, 0.3, False),
+    ((128,) * 8 + (77,), 2, 5, True, 0.3, False),
+    ((300,) * 7 + (1,), 2, 4, False, 0.3, False),
 ]
 
 
