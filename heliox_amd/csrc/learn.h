@@ -14,8 +14,9 @@
 //     Tick tau lives in slot tau % (K_len + 1), slot 0 starts as tick 0's, and the slot a
 //     tick writes is never in its own read window.  The dv/dw slices alternate between
 //     two buffers (the previous one is still read for dx).
-//     A per-slot fp32 scale carries the Frobenius clip's rescaling of the history
-//     instead of rewriting K_len slices.
+//     Each group of four columns of a slot has an fp32 scale: a power of two that keeps X
+//     in range, times the Frobenius clip's rescaling of the history (instead of rewriting
+//     K_len slices).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -91,7 +92,9 @@ struct ReplayCorrArgs {
     const float* x = nullptr;         // the ring of X slices
     long long xslice = 0;             // floats per slice
     const long long* xoff = nullptr;  // per block offset into a slice
-    const float* slot_scale = nullptr;
+    const float* xscale = nullptr;    // the ring of X's scales, one per group of four columns
+    const int* xgroup = nullptr;      // per block its first group
+    int xgroups = 0;                  // groups per slot
     int R = 1;                        // ring slots
     int h0 = 0;                       // slot of the window's first tick
     const float* kp = nullptr;
@@ -120,6 +123,16 @@ struct ReplayFinishArgs {
     ReplayDx dx;
 };
 
+// the exponents of X's groups for ticks 0 .. ticks - 1, and the ring's scales at 1
+struct ReplayRangeArgs {
+    int N = 0, ticks = 0, R = 1, xgroups = 0;
+    const int2* group_col = nullptr;  // first column and columns of each group
+    const float* dv = nullptr;        // dIt/dv and dIt/dvpre (T, N)
+    const float* dp = nullptr;
+    unsigned char* xdown = nullptr;   // (ticks, xgroups)
+    float* xscale = nullptr;          // (R, xgroups)
+};
+
 struct ReplayTickArgs {
     int N = 0;
     const float* cur = nullptr;       // the tick's slice
@@ -129,8 +142,7 @@ struct ReplayTickArgs {
     int npart = 0;
     float thr = 0.f;
     float* gs = nullptr;
-    float* slot_scale = nullptr;
-    int R = 1, cur_slot = 0;
+    int R = 1, cur_slot = 0;          // ring slots, this tick's
     float* tick_scale = nullptr;
     const int* po = nullptr;
     int n_out = 0;
@@ -138,6 +150,10 @@ struct ReplayTickArgs {
     float* w_tick = nullptr;
     float* dw_acc = nullptr;
     float* x = nullptr;               // slot of this tick (null: no X)
+    const unsigned char* xdown = nullptr;   // this tick's exponents
+    float* xscale = nullptr;          // the ring of scales
+    const int* col_group = nullptr;   // group of each column
+    int xgroups = 0;
     const long long* xoff = nullptr;
     const int* col_block = nullptr;
     const int* start = nullptr;
@@ -154,6 +170,7 @@ int rp_corr_row_tiles(int N);
 int rp_corr_splits(int N, int ntiles, int max_bnp, int tw);
 void launch_rp_finish(ReplayFinishArgs a, hipStream_t s);
 int rp_finish_blocks(int N);
+void launch_rp_range(const ReplayRangeArgs& a, hipStream_t s);
 void launch_rp_tick(ReplayTickArgs a, hipStream_t s);
 void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s);
 void launch_rp_scale_into(const float* src, float scale, float* dst, long long n, hipStream_t s);
@@ -227,9 +244,10 @@ public:
     long long corr_launches = 0;
 
     struct Workspace {
-        float *slices = nullptr, *x = nullptr, *part = nullptr, *base = nullptr, *slot_scale = nullptr, *gs = nullptr,
+        float *slices = nullptr, *x = nullptr, *part = nullptr, *base = nullptr, *xscale = nullptr, *gs = nullptr,
               *tick_scale = nullptr, *w_tick = nullptr, *dw_acc = nullptr, *dl = nullptr, *dx = nullptr,
               *dw_out = nullptr;
+        unsigned char* xdown = nullptr;
         int *po = nullptr, *pre = nullptr, *pin = nullptr;
         double* norm_part = nullptr;
         int base_ticks = 0;               // ticks base holds
@@ -245,7 +263,7 @@ private:
     // ways of providing them.
     struct Sizes {
         int R = 1;
-        size_t x = 0, part = 0, norm = 0;
+        size_t x = 0, xscale = 0, part = 0, norm = 0;
     };
     Sizes sizes_for(int N, bool percise) const;
 
@@ -258,8 +276,9 @@ private:
     std::vector<void*> blk_mem_;
     float* d_kp_ = nullptr;
     long long *d_koff_ = nullptr, *d_boff_ = nullptr, *d_xoff_ = nullptr;
-    int *d_start_ = nullptr, *d_bn_ = nullptr, *d_bnp_ = nullptr, *d_col_block_ = nullptr;
-    int2* d_tiles_ = nullptr;
+    int *d_start_ = nullptr, *d_bn_ = nullptr, *d_bnp_ = nullptr, *d_xgroup_ = nullptr, *d_col_block_ = nullptr,
+        *d_col_group_ = nullptr;
+    int2 *d_tiles_ = nullptr, *d_group_col_ = nullptr;
     // capture cache (T, N) per channel
     int cap_N_ = 0, cap_T_ = 0, cap_kmul_ = 0;
     bool cap_percise_ = false;

@@ -225,6 +225,7 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
 
     const int kg = tid % (kKC / 4), r0 = tid / (kKC / 4);     // group within the chunk, first row
     const float* Xb = A.x + static_cast<long long>(A.xoff[b]);
+    const int xgroup = A.xgroup[b];
     const float* Kb = A.kp + A.koff[b];
     typedef float f4 __attribute__((ext_vector_type(4)));
     f4 ra[S::GA], rb[S::GB];
@@ -234,11 +235,11 @@ __global__ void __launch_bounds__(CorrShape<TJ>::kT) k_rp_corr(ReplayCorrArgs A)
     auto fetch = [&](int c) {
         const int pos = c * (kKC / 4) + kg;
         const int u = pos / nb4;
-        const int k = (pos - u * nb4) * 4;
+        const int k4 = pos - u * nb4, k = k4 * 4;
         in = pos < total;
         int h = A.h0 + (in ? u : 0);
         if (h >= A.R) h -= A.R;
-        sig = A.slot_scale[h];
+        sig = A.xscale[h * A.xgroups + xgroup + (in ? k4 : 0)];
         const float* X = Xb + h * A.xslice + (in ? k : 0);
         const float* K = Kb + static_cast<size_t>(A.k_t0 + (in ? u : 0)) * bn * bnp + (in ? k : 0);
 #pragma unroll
@@ -417,14 +418,43 @@ __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
     }
 }
 
+// ---------------------------------------------------------------- X's range
+// X is formed before the clip factors of its own and of later ticks are known, so it has to
+// hold products that only those factors bring back into fp32's range.  Each 16-byte group
+// of columns keeps X 2^-down, down from the group's largest signal, and 2^down times the
+// factors so far meets it when the correction reads X.  |X 2^-down| stays at or below |D|
+// (but for signals and slices both above 2^126), and a power of two changes no bit of a
+// normal number; beside a signal of 2^e, its three neighbours lose what lies below
+// 2^(e - 148).  Cost at N = 2048: k_rp_corr 447.6 -> 449.4 us, k_rp_tick 16.3 -> 17.1; with
+// a scale per column, 16 bytes to read beside X's 16, k_rp_corr 452 to 455.  This kernel makes down for every tick and sets the
+// ring's scales to 1.
+__global__ void __launch_bounds__(kThreads) k_rp_range(ReplayRangeArgs A) {
+    const long long ndown = static_cast<long long>(A.ticks) * A.xgroups;
+    const long long n = ndown > static_cast<long long>(A.R) * A.xgroups ? ndown : static_cast<long long>(A.R) * A.xgroups;
+    for (long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x; i < n;
+         i += static_cast<long long>(gridDim.x) * kThreads) {
+        if (i < static_cast<long long>(A.R) * A.xgroups) A.xscale[i] = 1.f;
+        if (i >= ndown) continue;
+        const int t = static_cast<int>(i / A.xgroups), g = static_cast<int>(i - static_cast<long long>(t) * A.xgroups);
+        const size_t at = static_cast<size_t>(t + 1) * A.N + A.group_col[g].x;
+        int down = 0;
+        for (int c = 0; c < A.group_col[g].y; ++c) {
+            const float m = fmaxf(fabsf(A.dv[at + c]), fabsf(A.dp[at + c]));
+            if (m >= 0.25f && isfinite(m)) down = max(down, min(ilogbf(m) + 2, 127));
+        }
+        A.xdown[i] = static_cast<unsigned char>(down);
+    }
+}
+
 // ---------------------------------------------------------------- a tick's end
 // The Frobenius clip (replay_frobenius_*_kernel replay_dw_dx.cu:28-93, the driver's
 // decision LearnRuntime.cpp:2238-2262): l2 over the finite entries; above the threshold
 // the tick's slice, the history, the accumulators and the grad scale are all multiplied
 // by thr / l2.  Every workgroup that needs the factor sums the norm's partials itself, in
-// the same order (a launch of its own took 4 us); block 0 stores it with the rescaled
-// scales, which only later launches read.  w_tick (replay_dw_dx.cu:96-114): one wave per
-// row.  The remaining blocks form X of this tick from its slice.
+// the same order (a launch of its own took 4 us); block 0 stores it, and all rescale their
+// share of the history's scales, which only later launches read.  w_tick
+// (replay_dw_dx.cu:96-114): one wave per row.  The remaining blocks form X of this tick
+// from its slice.
 template <int kGather, class I>
 __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
     __shared__ double sh[kThreads];
@@ -446,8 +476,9 @@ __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
             }
             const int p = A.pre[c], b = A.col_block[c];
             const float g = p >= 0 ? A.cur[static_cast<size_t>(row) * N + p] : 0.f;
+            const int down = A.xdown[A.col_group[c]];
             A.x[A.xoff[b] + static_cast<size_t>(row) * A.bnp[b] + c - A.start[b]] =
-                A.cur[e] * A.dv[c] + g * A.dp[c];
+                A.cur[e] * ldexpf(A.dv[c], -down) + g * ldexpf(A.dp[c], -down);
         }
         return;
     }
@@ -463,9 +494,13 @@ __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
             *A.tick_scale = sc;
             if (sc != 1.f) *A.gs *= sc;
         }
-        for (int r = tid; r < A.R; r += kThreads) {
-            if (r == A.cur_slot) A.slot_scale[r] = sc;
-            else if (sc != 1.f) A.slot_scale[r] *= sc;
+    }
+    if (A.x) {                                                // the scales of X's groups
+        const int first = sc != 1.f ? 0 : A.cur_slot, last = sc != 1.f ? A.R : A.cur_slot + 1;
+        const int here = A.cur_slot * A.xgroups;
+        for (int q = first * A.xgroups + blockIdx.x * kThreads + tid; q < last * A.xgroups; q += A.wblocks * kThreads) {
+            const int g = q - here;
+            A.xscale[q] = g >= 0 && g < A.xgroups ? ldexpf(sc, A.xdown[g]) : A.xscale[q] * sc;
         }
     }
     const unsigned row = blockIdx.x * (kThreads / 64) + (tid >> 6);
@@ -580,6 +615,12 @@ void launch_rp_finish(ReplayFinishArgs a, hipStream_t s) {
             if (narrow_slice(a.O.N)) go(k_rp_finish<kFinishMost, unsigned>);
             else go(k_rp_finish<kFinishMost, unsigned long long>);
     }
+}
+
+void launch_rp_range(const ReplayRangeArgs& a, hipStream_t s) {
+    const long long n = static_cast<long long>(std::max(a.ticks, a.R)) * a.xgroups;
+    const long long blocks = std::min<long long>((n + kThreads - 1) / kThreads, 4096);
+    hipLaunchKernelGGL(k_rp_range, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, s, a);
 }
 
 void launch_rp_tick(ReplayTickArgs a, hipStream_t s) {

@@ -111,7 +111,8 @@ int LearnRuntime::set_dense_blocks(int nblk, const float* const* data, const int
     try {
         int start = 0, ncol = 0;
         long long koff = 0, boff = 0;
-        std::vector<int> bnp, col_block;
+        std::vector<int> bnp, xgroup, col_block, col_group;
+        std::vector<int2> group_col;
         for (int b = 0; b < nblk; ++b) ncol += bn[b];
         for (int b = 0; b < nblk; ++b) {
             const int n = bn[b], np = (n + 3) & ~3;
@@ -121,6 +122,11 @@ int LearnRuntime::set_dense_blocks(int nblk, const float* const* data, const int
             koff_.push_back(koff);
             boff_.push_back(boff);
             xoff_.push_back(static_cast<long long>(ncol) * xcols_);
+            xgroup.push_back(static_cast<int>(xcols_ / 4));
+            for (int k = 0; k < n; k += 4) {
+                col_group.insert(col_group.end(), std::min(4, n - k), static_cast<int>(group_col.size()));
+                group_col.push_back(make_int2(start + k, std::min(4, n - k)));
+            }
             col_block.insert(col_block.end(), n, b);
             max_bn_ = std::max(max_bn_, n);
             max_bnp_ = std::max(max_bnp_, np);
@@ -152,6 +158,9 @@ int LearnRuntime::set_dense_blocks(int nblk, const float* const* data, const int
         d_koff_ = lupload(blk_mem_, koff_.data(), koff_.size());
         d_boff_ = lupload(blk_mem_, boff_.data(), boff_.size());
         d_xoff_ = lupload(blk_mem_, xoff_.data(), xoff_.size());
+        d_xgroup_ = lupload(blk_mem_, xgroup.data(), xgroup.size());
+        d_col_group_ = lupload(blk_mem_, col_group.data(), col_group.size());
+        d_group_col_ = lupload(blk_mem_, group_col.data(), group_col.size());
         d_start_ = lupload(blk_mem_, start_.data(), start_.size());
         d_bn_ = lupload(blk_mem_, bn_.data(), bn_.size());
         d_bnp_ = lupload(blk_mem_, bnp.data(), bnp.size());
@@ -312,7 +321,8 @@ int LearnRuntime::replay(const ReplayIn& in) {
             ws_.part = lalloc<float>(ws_mem_, z.part);
             ws_.base_ticks = kBaseTicks;
             ws_.base = lalloc<float>(ws_mem_, static_cast<size_t>(base_len_) * kBaseTicks);
-            ws_.slot_scale = lalloc<float>(ws_mem_, z.R);
+            ws_.xscale = lalloc<float>(ws_mem_, z.xscale);
+            ws_.xdown = lalloc<unsigned char>(ws_mem_, z.xscale ? static_cast<size_t>(ks) * xcols_ / 4 : 0);
             ws_.gs = lalloc<float>(ws_mem_, 1);
             ws_.tick_scale = lalloc<float>(ws_mem_, 1);
             ws_.w_tick = lalloc<float>(ws_mem_, N);
@@ -345,6 +355,7 @@ LearnRuntime::Sizes LearnRuntime::sizes_for(int N, bool percise) const {
     if (percise) {
         const int splits = rp_corr_splits(N, ntiles, max_bnp_, k_len_);   // the most any window takes
         z.x = static_cast<size_t>(z.R) * N * xcols_;
+        z.xscale = static_cast<size_t>(z.R) * xcols_ / 4;
         z.part = splits > 1 ? static_cast<size_t>(splits) * N * N : 0;
     }
     return z;
@@ -369,7 +380,20 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
         if (need_dx) LRC(hipMemcpyAsync(ws.pin, in.pin, sizeof(int) * in.n_in, hipMemcpyHostToDevice, stream_));
 
         launch_fill_f32(ws.slices, 0.f, static_cast<long long>(slice), stream_);      // tick 0
-        launch_fill_f32(ws.slot_scale, 1.f, R, stream_);
+        const int xgroups = static_cast<int>(xcols_ / 4);
+        if (in.percise) {
+            ReplayRangeArgs G{};
+            G.N = N;
+            G.ticks = ks;
+            G.R = R;
+            G.xgroups = xgroups;
+            G.group_col = d_group_col_;
+            G.dv = sig[1];
+            G.dp = sig[2];
+            G.xdown = ws.xdown;
+            G.xscale = ws.xscale;
+            launch_rp_range(G, stream_);
+        }
         launch_fill_f32(ws.gs, static_cast<float>(in.grad_scale), 1, stream_);
         launch_fill_f32(ws.tick_scale, 1.f, 1, stream_);
         launch_fill_f32(ws.dw_acc, 0.f, N, stream_);
@@ -387,7 +411,9 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
         K.norm_part = ws.norm_part;
         K.thr = thr;
         K.gs = ws.gs;
-        K.slot_scale = ws.slot_scale;
+        K.xscale = ws.xscale;
+        K.col_group = d_col_group_;
+        K.xgroups = xgroups;
         K.R = R;
         K.tick_scale = ws.tick_scale;
         K.po = ws.po;
@@ -403,6 +429,7 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
         auto with_x = [&](int t) {
             const bool need = in.percise && t < ks;
             K.x = need ? ws.x + static_cast<size_t>(t % R) * xslice : nullptr;
+            K.xdown = need ? ws.xdown + static_cast<size_t>(t) * xgroups : nullptr;
             K.dv = need ? sig[1] + static_cast<size_t>(t + 1) * N : nullptr;
             K.dp = need ? sig[2] + static_cast<size_t>(t + 1) * N : nullptr;
         };
@@ -463,7 +490,9 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
                 C.x = ws.x;
                 C.xslice = xslice;
                 C.xoff = d_xoff_;
-                C.slot_scale = ws.slot_scale;
+                C.xscale = ws.xscale;
+                C.xgroup = d_xgroup_;
+                C.xgroups = xgroups;
                 C.R = R;
                 C.h0 = (t_lr - tw) % R;
                 C.kp = d_kp_;
@@ -621,7 +650,8 @@ int LearnRuntime::replay_from_host_noalloc(const ReplayIn& in, const float* it_n
             w.part = c.take<float>(z.part);
             w.base_ticks = base_ticks;
             w.base = c.take<float>(static_cast<size_t>(base_len_) * base_ticks);
-            w.slot_scale = c.take<float>(z.R);
+            w.xscale = c.take<float>(z.xscale);
+            w.xdown = c.take<unsigned char>(z.xscale ? static_cast<size_t>(ks) * xcols_ / 4 : 0);
             w.gs = c.take<float>(1);
             w.tick_scale = c.take<float>(1);
             w.w_tick = c.take<float>(N);
