@@ -339,7 +339,8 @@ struct hx_sim {
     // Solve by substructuring (k_solve_split): in use when no cell has more than
     // kSplitMaxChunks chunks and the model no more than kSplitMaxTotal.  It leaves the assembled matrix in d and rhs; the pivots and
     // the solution go there when something reads them (make_dx): after every solve once a
-    // handle, monitor or transfer names d or rhs (need_dx), else from the call's last step
+    // handle, monitor, transfer or VecPlay names d or rhs (need_dx; the last writes into them
+    // after the solve), else from the call's last step
     // (dx_pending, with its form in dx_yform and its old voltages in d_vold).
     bool solve_split_allowed = true;
     bool solve_split = false;
@@ -3694,6 +3695,7 @@ int hx_load_model(hx_sim* sim) {
     for (auto& vp : sim->vecplay) {
         Ref r = sim->resolve(vp.mech, vp.var, vp.idx);
         if (!r.dev) return sim->fail("vecplay target %s.%s[%d] not found", vp.mech.c_str(), vp.var.c_str(), vp.idx);
+        sim->note_dx_reader(r);
         vp.target = r.dev;
     }
     for (size_t i = 0; i < sim->mon_name.size(); ++i) {
@@ -4133,6 +4135,7 @@ int hx_add_vecplay(hx_sim* sim, const char* mech, const char* var, int idx, int 
         API_BEGIN
         Ref r = sim->resolve(mech, var, idx);
         if (!r.dev) return sim->fail("vecplay target %s.%s[%d] not found", mech, var, idx);
+        sim->note_dx_reader(r);
         vp.target = r.dev;
         API_END
     }

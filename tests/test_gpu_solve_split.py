@@ -115,3 +115,25 @@ def test_pivots_and_solution_on_demand(gpu_lib):
         assert np.array_equal(held.get_array("global", k), want), k
         assert np.array_equal(late.get_array("global", k), want), k
     assert held.get_variables_by_handles([0])[0] == plain.get_variable_value("global", "rhs", 5)
+
+
+def test_vecplay_into_the_solution(gpu_lib):
+    """VecPlay writes its rhs entry after each solve; the other entries stay the solution's."""
+    spec = passive(bushy(60), 4, False)
+    print("case split vecplay into rhs", flush=True)
+    out = []
+    for split in (True, False):
+        for late in (False, True):
+            g = Sim()
+            g.set_solve_split(split)
+            g.load_model_from_spec(spec, add_monitors=False)
+            g.finitialize(-65.0)
+            if late:
+                g.continue_run(0.5)
+            assert g.add_vecplay("global", "rhs", 7, [0.0, 100.0], [3.0, 3.0]) == 0
+            g.continue_run(0.5 if late else 1.0)
+            out.append((g.get_array("global", "d"), g.get_array("global", "rhs")))
+    for d, rhs in out:
+        assert rhs[7] == 3.0
+        np.testing.assert_allclose(d, out[2][0], rtol=TOL)
+        assert float(np.max(np.abs(rhs - out[2][1]))) < TOL
