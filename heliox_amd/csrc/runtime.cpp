@@ -339,8 +339,8 @@ struct hx_sim {
     // Solve by substructuring (k_solve_split): in use when no cell has more than
     // kSplitMaxChunks chunks and the model no more than kSplitMaxTotal.  It leaves the assembled matrix in d and rhs; the pivots and
     // the solution go there when something reads them (make_dx): after every solve once a
-    // handle, monitor, transfer or VecPlay names d or rhs (need_dx; the last writes into them
-    // after the solve), else from the call's last step
+    // monitor, captured signal, transfer, optimizer or VecPlay names d or rhs (need_dx; the
+    // last writes into them after the solve), else from the call's last step
     // (dx_pending, with its form in dx_yform and its old voltages in d_vold).
     bool solve_split_allowed = true;
     bool solve_split = false;
@@ -3975,7 +3975,6 @@ int hx_get_variable_handle(hx_sim* sim, const char* mech, const char* var, int i
     Ref r = sim->resolve(mech ? mech : "", var ? var : "", idx);
     if (!r.dev) return sim->fail("variable %s.%s[%d] not found", mech, var, idx);
     if (r.klass == 1) sim->write_assigned = true;
-    sim->note_dx_reader(r);
     sim->handles.push_back(r);
     return static_cast<int>(sim->handles.size()) - 1;
     API_END
@@ -3985,6 +3984,7 @@ int hx_get_variable_by_handle(hx_sim* sim, int h, double* out) {
     HX_SETTLE(sim);
     if (h < 0 || h >= static_cast<int>(sim->handles.size()) || !out) return sim->fail("bad variable handle");
     API_BEGIN
+    if (sim->reads_dx(sim->handles[h])) sim->make_dx();
     HXC(hipStreamSynchronize(sim->stream));
     HXC(hipMemcpy(out, sim->handles[h].dev, sizeof(double), hipMemcpyDeviceToHost));
     return 0;
@@ -3995,6 +3995,7 @@ int hx_set_variable_by_handle(hx_sim* sim, int h, double value) {
     HX_SETTLE(sim);
     if (h < 0 || h >= static_cast<int>(sim->handles.size())) return sim->fail("bad variable handle");
     API_BEGIN
+    if (sim->reads_dx(sim->handles[h])) sim->make_dx();
     HXC(hipStreamSynchronize(sim->stream));
     HXC(hipMemcpy(sim->handles[h].dev, &value, sizeof(double), hipMemcpyHostToDevice));
     sim->mirror_ab(sim->handles[h], value);
@@ -5184,6 +5185,7 @@ int hx_optimizer_add_param_batch(hx_sim* sim, int opt, int n, const int* weight_
     if (opt < 0 || opt >= static_cast<int>(sim->adams.size())) return sim->fail("optimizer %d not found", opt);
     if (n <= 0 || !weight_handles || !grad_handles)
         return sim->fail("optimizer_add_param_batch: handle lists must be non-empty and have equal length");
+    API_BEGIN
     std::vector<double*> w(n), g(n);
     const int nh = static_cast<int>(sim->handles.size());
     for (int i = 0; i < n; ++i) {
@@ -5193,8 +5195,11 @@ int hx_optimizer_add_param_batch(hx_sim* sim, int opt, int n, const int* weight_
             return sim->fail("optimizer_add_param_batch: invalid grad handle %d", grad_handles[i]);
         w[i] = sim->handles[weight_handles[i]].dev;
         g[i] = sim->handles[grad_handles[i]].dev;
+        sim->note_dx_reader(sim->handles[weight_handles[i]]);
+        sim->note_dx_reader(sim->handles[grad_handles[i]]);
     }
     return sim->opt_add_group(opt, w, g, impedance);
+    API_END
 }
 
 int hx_optimizer_add_param(hx_sim* sim, int opt, int weight_handle, int grad_handle, double impedance) {
@@ -5230,6 +5235,7 @@ int hx_optimizer_add_external_grads(hx_sim* sim, int opt, int n, const int* weig
     o.d_ext = dalloc<double>(sim->owned, n);
     o.n_ext = n;
     HXC(hipMemset(o.d_ext, 0, sizeof(double) * n));
+    for (int i = 0; i < n; ++i) sim->note_dx_reader(sim->handles[weight_handles[i]]);
     for (int i = 0; i < n; ++i)      // one group per weight (SimWrapper.cpp:284-353)
         sim->opt_add_group(opt, {sim->handles[weight_handles[i]].dev}, {o.d_ext + i}, impedance);
     return 0;

@@ -117,6 +117,33 @@ def test_pivots_and_solution_on_demand(gpu_lib):
     assert held.get_variables_by_handles([0])[0] == plain.get_variable_value("global", "rhs", 5)
 
 
+def test_handles_and_monitors_of_the_solution(gpu_lib):
+    """Handles of d and rhs read after every step, one written, and a monitor of rhs: the
+    values of the arrays after the same steps."""
+    spec = passive(bushy(60), 4, False)
+    print("case split handles", flush=True)
+    names = [("global", "rhs", 5), ("global", "d", 70)]
+    held, plain, watched, rounds = run(spec, True), run(spec, True), run(spec, True), run(spec, False)
+    hs = [held.get_variable_handle(*n) for n in names]
+    m = [g.add_monitor(*names[0]) for g in (watched, rounds)]
+    for _ in range(3):
+        for g in (held, plain, watched, rounds):
+            g.fadvance()
+        got = held.get_variables_by_handles(hs)
+        want = [plain.get_array("global", "rhs")[5], plain.get_array("global", "d")[70]]
+        assert list(got) == want
+        assert watched.get_variable_value(*names[0]) == want[0]
+    a, b = watched.monitor_array(m[0]), rounds.monitor_array(m[1])
+    assert a.size == b.size > 0 and float(np.max(np.abs(a - b))) < TOL and np.any(b != 0)
+    held.fadvance()
+    plain.fadvance()
+    held.set_variable_by_handle(hs[0], 2.5)
+    rhs = plain.get_array("global", "rhs")
+    rhs[5] = 2.5
+    assert np.array_equal(held.get_array("global", "rhs"), rhs)
+    assert np.array_equal(held.get_array("global", "d"), plain.get_array("global", "d"))
+
+
 def test_vecplay_into_the_solution(gpu_lib):
     """VecPlay writes its rhs entry after each solve; the other entries stay the solution's."""
     spec = passive(bushy(60), 4, False)
