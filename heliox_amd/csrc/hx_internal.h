@@ -208,19 +208,10 @@ struct alignas(16) SplitDesc {
     uint8_t child_count;
 };
 static_assert(sizeof(SplitDesc) == 16, "SplitDesc must stay 16 bytes");
-// A cell of more chunks (three wavefronts a SIMD at 168 registers) is left to the round-by-round solve; a
-// pack stops taking cells at kSplitPackChunks (two wavefronts).
+// A cell of more chunks (12 wavefronts, what a CU holds) is left to the round-by-round
+// solve; a pack stops taking cells at kSplitPackChunks (two wavefronts).
 constexpr int kSplitMaxChunks = 768;
 constexpr int kSplitPackChunks = 128;
-// The chunks the chip holds at once (256 CUs, 12 wavefronts of this kernel's registers).  A
-// model of more has workgroups queueing, and the rounds, which leave room for the other
-// group's node pass beside them, catch up: for cells whose rounds are held in LDS at about
-// this many (100 steps of 500-node trees: 1500 cells, 80k chunks, 10.4 -> 7.7 ms; 3000,
-// 161k, 12.8 -> 11.8; 6000, 322k, 22.3 -> 25.6), for larger, streamed cells past twice as
-// many (5000-node pyramidal cells: 300, 185k, 19.0 -> 12.8 ms; 600, 371k, 28.8 -> 25.6;
-// 1000, 619k, even; 2000, 1.24M, 0.52 -> 0.64 ms a step).  A rule on the model's chunks and
-// largest cell, not its packs, so that no choice of units or groups changes the route.
-constexpr long long kSplitMaxTotal = 256LL * 12 * kWave;
 struct SplitArgs {
     const SplitDesc* desc;        // [npack * threads]
     const int* levels;            // [npack * lev_stride]: level count, then the first slot of each level and the end

@@ -336,9 +336,8 @@ struct hx_sim {
     bool solve_voltage_allowed = true;   // the solve may take rhs + d v and yield v_new itself
     bool solve_voltage = false;          // in use: every d and rhs term of a step is the node kernel's
     int pass_yform = 0;                  // the node pass being launched stores rhs + d v
-    // Solve by substructuring (k_solve_split): in use when no cell has more than
-    // kSplitMaxChunks chunks and the model no more than kSplitMaxTotal.  It leaves the assembled matrix in d and rhs; the pivots and
-    // the solution go there when something reads them (make_dx): after every solve once a
+    // Solve by substructuring (k_solve_split): in use where build_packs says so.  It leaves
+    // the assembled matrix in d and rhs; the pivots and the solution go there when something reads them (make_dx): after every solve once a
     // monitor, captured signal, transfer, optimizer or VecPlay names d or rhs (need_dx; the
     // last writes into them after the solve), else from the call's last step
     // (dx_pending, with its form in dx_yform and its old voltages in d_vold).
@@ -347,18 +346,22 @@ struct hx_sim {
     bool need_dx = false, dx_pending = false;
     int dx_yform = 0;
     double* d_vold = nullptr;
-    std::vector<SplitDesc> split_descs;
-    std::vector<int> split_levels, unit_pack_begin;
-    int split_threads = 0, split_lev_stride = 0;
-    SplitDesc* d_split_desc = nullptr;
-    int* d_split_levels = nullptr;
+    // the packs of one workgroup size, one launch; those of unit u are
+    // [unit_begin[u], unit_begin[u + 1])
+    struct SplitClass {
+        int threads = 0, lev_stride = 0;
+        std::vector<int> unit_begin;
+        SplitDesc* d_desc = nullptr;
+        int* d_levels = nullptr;
+    };
+    std::vector<SplitClass> split_classes;
     // A taped run in the voltage form keeps the rounds: its gradients are sums of terms that
     // cancel, and carry the rounding of the solve 1000 times enlarged (12 pyramidal cells,
     // 100 steps, against 64 bits: 3.7e-11 with the rounds, 5.6e-11 without).
     bool use_split() const { return solve_split && !(tape_on && solve_voltage); }
     void build_packs();
     SolveArgs solve_args(int unit0, int unit1, bool store) const;
-    SplitArgs split_args(int unit0, int unit1) const;
+    SplitArgs split_args(const SplitClass& c, int unit0, int unit1) const;
     void issue_solve(int unit0, int unit1, hipStream_t s);
     bool reads_dx(const Ref& r) const {
         return d_d && ((r.dev >= d_d && r.dev < d_d + nnode) || (r.dev >= d_rhs && r.dev < d_rhs + nnode));
@@ -981,7 +984,6 @@ void hx_sim::build_layout() {
         U = std::max(1, U / 2);
     }
     unit_cells = U;
-    build_packs();
 
     // mechanism instance order: by solver-order node (stable); artificial cells
     // sit on no node and keep their own order
@@ -1047,21 +1049,38 @@ void hx_sim::build_layout() {
 // The packs of k_solve_split: each unit's cells in order, as many to a pack as fit
 // kSplitPackChunks (one at least).  A unit's chunk slots are breadth-first over all its
 // cells, so the slots of a few of them in the same order are breadth-first too.
+//
+// The route, from the model's cells alone (no choice of units or groups changes it, which
+// would change the voltages' last bits): the kernel's wavefronts are counted in passes, what
+// the chip holds at once (256 CUs; 12 wavefronts of the voltage form's 157 registers, 8 of
+// the change form's 184, 12 of its 768-thread instance).  A launch of more than a pass has
+// workgroups queueing, and the rounds, which leave room for the other group's node pass
+// beside them, catch up: at one pass where something couples the cells (one group, one
+// launch), at 1.7 otherwise (two groups), and one later where the rounds are streamed from
+// HBM (87 us a step for 5000-node cells).  us a step, split and rounds:
+//   one group, change form: 12000 101-node cells (0.82 passes) 33, 40; 16000 (1.1) 53, 43;
+//     200-node network, 6000 cells (0.96) 72, 77; 8000 (1.3) 101, 88;
+//   two groups, change form: 4000 500-node cells (1.64) 86, 92; 5000 (2.05) 118, 97;
+//   two groups, voltage form: 5000 500-node cells (1.38) 60, 68; 6500 (1.8) 75, 70;
+//   one group, 5000-node cells: 500 (1.95) 94, 112; 600 (2.3) 125, 114;
+//   two groups, voltage form, 5000-node cells: 600 (2.3) 171, 213; 1000 (3.9) even;
+//   one 5000-node cell, one group, and 20000 of 101 nodes (1.4) 94, 100; 40000 (2.75) 131, 115.
 void hx_sim::build_packs() {
-    split_descs.clear();
-    split_levels.clear();
-    unit_pack_begin.assign(nunit + 1, 0);
-    split_threads = split_lev_stride = 0;
+    split_classes.clear();
     solve_split = false;
     struct Pack {
+        int unit;
         std::vector<SplitDesc> desc;     // by thread
         std::vector<int> lev;            // first slot of each level, then the end
     };
+    // wavefronts a CU holds for a workgroup of this many chunks
+    auto waves_of = [](int chunks) { return (chunks + kWave - 1) / kWave; };
+    auto cu_waves = [&](int chunks) { return solve_voltage || chunks > 512 ? 12 : 8; };
     std::vector<Pack> packs;
-    size_t max_lev = 0;
+    double passes = 0.0;
     int max_chunks = 0, max_nodes = 0;
     for (int u = 0; u < nunit; ++u) {
-        unit_pack_begin[u] = static_cast<int>(packs.size());
+        const int pack0 = static_cast<int>(packs.size());
         const int nc = unit_desc_begin[u + 1] - unit_desc_begin[u];
         // by slot: the chunk's descriptor, head and round, its cell (of the unit) and level
         std::vector<const ChunkDesc*> cd(nc, nullptr);
@@ -1094,25 +1113,25 @@ void hx_sim::build_packs() {
         int fill = 0;
         for (size_t c = 0; c < chunks_of.size(); ++c) {
             if (chunks_of[c] > kSplitMaxChunks) return;
+            // small cells share wavefronts; a larger one takes its share of a CU
+            passes += chunks_of[c] <= kSplitPackChunks
+                          ? static_cast<double>(chunks_of[c]) / (256 * kWave * cu_waves(kSplitPackChunks))
+                          : 1.0 / (256 * (cu_waves(chunks_of[c]) / waves_of(chunks_of[c])));
             if (c == 0 || fill + chunks_of[c] > kSplitPackChunks) {
-                packs.emplace_back();
+                packs.push_back({u, {}, {}});
                 fill = 0;
             }
             fill += chunks_of[c];
             pack_of[c] = static_cast<int>(packs.size()) - 1;
             max_chunks = std::max(max_chunks, fill);
         }
-        std::vector<int> slot(nc), used(packs.size() - unit_pack_begin[u], 0);
+        std::vector<int> slot(nc), used(packs.size() - pack0, 0);
         for (int q = 0; q < nc; ++q) {
             Pack& p = packs[pack_of[cell[q]]];
-            slot[q] = used[pack_of[cell[q]] - unit_pack_begin[u]]++;
+            slot[q] = used[pack_of[cell[q]] - pack0]++;
             if (level[q] == static_cast<int>(p.lev.size())) p.lev.push_back(slot[q]);
         }
-        for (size_t i = 0; i < used.size(); ++i) {
-            Pack& p = packs[unit_pack_begin[u] + i];
-            p.lev.push_back(used[i]);
-            max_lev = std::max(max_lev, p.lev.size());
-        }
+        for (size_t i = 0; i < used.size(); ++i) packs[pack0 + i].lev.push_back(used[i]);
         for (int q : order) {
             SplitDesc d{};
             d.base = base[q];
@@ -1125,22 +1144,50 @@ void hx_sim::build_packs() {
             packs[pack_of[cell[q]]].desc.push_back(d);
         }
     }
-    unit_pack_begin[nunit] = static_cast<int>(packs.size());
-    split_threads = (max_chunks + kWave - 1) / kWave * kWave;
-    split_lev_stride = static_cast<int>(max_lev) + 1;
-    for (const Pack& p : packs) {
-        for (int i = 0; i < split_threads; ++i) {
-            SplitDesc d = p.desc[0];         // a thread past the pack's chunks reads a head and writes nothing
-            d.slot = d.parent = kNone;
-            split_descs.push_back(i < static_cast<int>(p.desc.size()) ? p.desc[i] : d);
-        }
-        split_levels.push_back(static_cast<int>(p.lev.size()) - 1);
-        for (int i = 0; i + 1 < split_lev_stride; ++i)
-            split_levels.push_back(i < static_cast<int>(p.lev.size()) ? p.lev[i] : p.lev.back());
-    }
     const bool resident_cells = static_cast<size_t>(max_nodes) * kStageArrays * sizeof(double) <= kResUnitBudget;
     solve_split = solve_split_allowed && !packs.empty() &&
-                  static_cast<long long>(descs.size()) <= (resident_cells ? 1 : 2) * kSplitMaxTotal;
+                  passes <= (groups_coupled ? 1.0 : 1.7) + (resident_cells ? 0.0 : 1.0);
+    if (!solve_split) return;
+    // A launch has one workgroup size.  One launch for all packs while they run in two
+    // passes of the largest (1 pyramidal cell beside 200 101-node cells: 39 us a step, 47
+    // with a launch per class; 5 and 500 500-node cells: 52 and 55), else one for each class
+    // (1 and 1000: 63 and 52; 5 and 1500: 104 and 68; 20 and 16000 101-node cells: 140, 88).
+    const int most = 256 * std::max(1, cu_waves(max_chunks) / waves_of(max_chunks));
+    std::vector<int> bounds{kSplitPackChunks, 2 * kSplitPackChunks, 4 * kSplitPackChunks, kSplitMaxChunks};
+    if (static_cast<int>(packs.size()) <= 2 * most) bounds = {kSplitMaxChunks};
+    for (size_t k = 0; k < bounds.size(); ++k) {
+        auto size_of = [](const Pack& p) { return static_cast<int>(p.desc.size()); };
+        auto in = [&](const Pack& p) { return size_of(p) <= bounds[k] && (k == 0 || size_of(p) > bounds[k - 1]); };
+        SplitClass cl;
+        size_t max_lev = 0;
+        for (const Pack& p : packs)
+            if (in(p)) {
+                cl.threads = std::max(cl.threads, waves_of(size_of(p)) * kWave);
+                max_lev = std::max(max_lev, p.lev.size());
+            }
+        if (cl.threads == 0) continue;
+        cl.lev_stride = static_cast<int>(max_lev) + 1;
+        cl.unit_begin.assign(nunit + 1, 0);
+        std::vector<SplitDesc> out;
+        std::vector<int> levels;
+        for (const Pack& p : packs) {
+            if (!in(p)) continue;
+            ++cl.unit_begin[p.unit + 1];
+            for (int i = 0; i < cl.threads; ++i) {
+                SplitDesc d = p.desc[0];         // a thread past the pack's chunks reads a head and writes nothing
+                d.slot = d.parent = kNone;
+                out.push_back(i < size_of(p) ? p.desc[i] : d);
+            }
+            levels.push_back(static_cast<int>(p.lev.size()) - 1);
+            for (int i = 0; i + 1 < cl.lev_stride; ++i)
+                levels.push_back(i < static_cast<int>(p.lev.size()) ? p.lev[i] : p.lev.back());
+        }
+        for (int u = 0; u < nunit; ++u) cl.unit_begin[u + 1] += cl.unit_begin[u];
+        cl.d_desc = dupload(owned, out);
+        cl.d_levels = dupload(owned, levels);
+        split_classes.push_back(cl);
+    }
+    d_vold = dalloc<double>(owned, nnode);
 }
 
 static const int kSparseOrder[] = {M_PAS, M_NA_ION, M_K_ION, M_HH, M_CA_ION, M_CADYN, M_CAHVA, M_HDLA};
@@ -1220,11 +1267,6 @@ void hx_sim::upload() {
     d_rounds = dupload(owned, rounds);
     d_desc = dupload(owned, descs);
     need_dx = dx_pending = false;
-    if (solve_split) {
-        d_split_desc = dupload(owned, split_descs);
-        d_split_levels = dupload(owned, split_levels);
-        d_vold = dalloc<double>(owned, nnode);
-    }
     {
         int dev = 0;
         hipDeviceProp_t prop;
@@ -1589,6 +1631,7 @@ void hx_sim::upload() {
     d_spk_count = dalloc<int>(owned, 1);
     HXC(hipMemset(d_spk_count, 0, sizeof(int)));
     build_groups(vs_fo, ntgt);
+    build_packs();
 
     // gap transfers.  The reference copies them one after the other, so a HalfGap instance
     // named by several gaps ends with the last one's source; the transfer kernel copies
@@ -2669,14 +2712,14 @@ SolveArgs hx_sim::solve_args(int unit0, int unit1, bool store) const {
     return S;
 }
 
-SplitArgs hx_sim::split_args(int unit0, int unit1) const {
+SplitArgs hx_sim::split_args(const SplitClass& c, int unit0, int unit1) const {
     SplitArgs P{};
-    const int p0 = unit_pack_begin[unit0];
-    P.npack = unit_pack_begin[unit1] - p0;
-    P.threads = split_threads;
-    P.lev_stride = split_lev_stride;
-    P.desc = d_split_desc + static_cast<size_t>(p0) * split_threads;
-    P.levels = d_split_levels + static_cast<size_t>(p0) * split_lev_stride;
+    const int p0 = c.unit_begin[unit0];
+    P.npack = c.unit_begin[unit1] - p0;
+    P.threads = c.threads;
+    P.lev_stride = c.lev_stride;
+    P.desc = c.d_desc + static_cast<size_t>(p0) * c.threads;
+    P.levels = c.d_levels + static_cast<size_t>(p0) * c.lev_stride;
     P.rounds = d_rounds;
     P.v = d_v;
     P.d = d_d;
@@ -2694,7 +2737,7 @@ void hx_sim::issue_solve(int unit0, int unit1, hipStream_t s) {
         launch_solve(solve_args(unit0, unit1, store_dx()), max_slots, s);
         return;
     }
-    launch_solve_split(split_args(unit0, unit1), s);
+    for (const SplitClass& c : split_classes) launch_solve_split(split_args(c, unit0, unit1), s);
     if (need_dx) {
         SolveArgs S = solve_args(unit0, unit1, true);
         S.v = d_vold;
@@ -4627,6 +4670,7 @@ long long hx_get_info(hx_sim* sim, const char* key) {
     if (k == "solve_waves") return sim->solve_waves;
     if (k == "solve_resident") return sim->res_nodes > 0 ? 1 : 0;
     if (k == "solve_split") return sim->solve_split ? 1 : 0;
+    if (k == "solve_split_launches") return sim->solve_split ? static_cast<long long>(sim->split_classes.size()) : 0;
     if (k == "solve_voltage") return sim->solve_voltage ? 1 : 0;
     if (k == "nchunk_total") return static_cast<long long>(sim->descs.size());
     if (k == "event_slots") return sim->groups.empty() ? 0 : sim->groups[0].ring.nslot;
@@ -4962,18 +5006,20 @@ int hx_adjoint(hx_sim* sim, int nloss, const int* loss_nodes, const double* targ
     S.a = sim->d_sb;
     S.b = sim->d_sa;
     S.yform = 1;
-    SplitArgs P{};
     const bool split = sim->use_split();
-    if (split) {
-        P = sim->split_args(0, sim->nunit);
-        P.v = S.v;
-        P.d = S.d;
-        P.rhs = S.rhs;
-        P.a = S.a;
-        P.b = S.b;
-        P.yform = 1;
-        P.store_vold = 0;
-    }
+    std::vector<SplitArgs> split_solves;           // of the classes
+    if (split)
+        for (const auto& c : sim->split_classes) {
+            SplitArgs P = sim->split_args(c, 0, sim->nunit);
+            P.v = S.v;
+            P.d = S.d;
+            P.rhs = S.rhs;
+            P.a = S.a;
+            P.b = S.b;
+            P.yform = 1;
+            P.store_vold = 0;
+            split_solves.push_back(P);
+        }
     double* lv = sim->d_lv;
     double* lv2 = sim->d_lv2;
     const size_t row = static_cast<size_t>(N);
@@ -4995,7 +5041,8 @@ int hx_adjoint(hx_sim* sim, int nloss, const int* loss_nodes, const double* targ
         A.loss_v = (d_lmap && n >= 1) ? sim->d_tape_v + (n - 1) * row : nullptr;
         A.loss_tgt = n >= 1 ? d_tgt + static_cast<size_t>(n - 1) * nloss : nullptr;
         launch_adj_before_solve(A, st);
-        if (split) launch_solve_split(P, st);
+        if (split)
+            for (const SplitArgs& P : split_solves) launch_solve_split(P, st);
         else launch_solve(S, sim->max_slots, st);
         launch_adj_after_solve(A, st);
         if (n >= 1 && !d_lmap)

@@ -322,11 +322,14 @@ int hx_set_solve_waves(hx_sim* sim, int waves);
 int hx_set_solve_resident(hx_sim* sim, int enable);
 /* Tree solve by substructuring (no counterpart in the reference): enable = 1 (default) lets
  * every unbranched run of up to 16 nodes eliminate its interior at once, one thread each,
- * and solves the tree of the runs' tails level by level, where no cell has more than 768
- * such runs and the model no more than 196608 (393216 with cells above 1024 nodes); 0
- * solves round by round (hx_set_solve_resident), which also yields d and rhs after a step
- * in either case.  The two agree to rounding.  hx_get_info("solve_split") reports the
- * choice.  Call before hx_load_model. */
+ * and solves the tree of the runs' tails level by level.  In use where no cell has more than
+ * 768 such runs and the model is no larger than its cells' sizes and coupling let the GPU
+ * hold about at once (some 130000 runs of cells that share a launch, 330000 of independent
+ * ones).  0 solves round by round (hx_set_solve_resident), which also yields d and rhs after
+ * a step in either case; a monitor, captured signal, transfer, optimizer or VecPlay entry
+ * that names d or rhs runs both on every step.  The two agree to rounding: their voltages
+ * differ in the last bits.  hx_get_info("solve_split") reports the choice (fixed at load)
+ * and "solve_split_launches" the launches of a solve.  Call before hx_load_model. */
 int hx_set_solve_split(hx_sim* sim, int enable);
 /* Tree solve unknown (no counterpart in the reference): enable = 1 (default) lets a model
  * whose node kernel makes every term of d and rhs (no density mechanism on its own kernel,

@@ -1,8 +1,9 @@
 """The tree solve by substructuring (k_solve_split) against the round-by-round solve and the
 oracle, at the sizes where it could go wrong: cells of a single node, of one chunk and one
 more, packs of several cells, a level wider than a wavefront, more chunks than 512 threads
-and more than the kernel takes; with the voltage and with the change as the unknown; the
-pivots and the solution read after a step, through a handle, and after a coefficient changed."""
+and more than the kernel takes, cells of unequal size; with the voltage and with the change
+as the unknown; the pivots and the solution read after a step, through a handle, and after a
+coefficient changed."""
 import dataclasses
 
 import numpy as np
@@ -35,18 +36,22 @@ def bushy(n):
 
 
 def passive(parents, ncell, clamp):
-    """`ncell` copies of one tree with unequal couplings, pas everywhere; `clamp` adds a current
+    """`ncell` copies of one tree (see forest)."""
+    return forest([parents] * ncell, clamp)
+
+
+def forest(trees, clamp):
+    """Cells of these trees with unequal couplings, pas everywhere; `clamp` adds a current
     injection, which leaves the change as the unknown."""
-    m, n = len(parents), len(parents) * ncell
-    node = np.empty((ncell, m), np.int64)
-    node[:, 0] = np.arange(ncell)
-    node[:, 1:] = ncell + np.arange(ncell * (m - 1)).reshape(ncell, m - 1)
-    par = np.full(n, -1, np.int32)
-    for c in range(ncell):
-        par[node[c, 1:]] = node[c, np.asarray(parents[1:], np.int64)]
-    rng = np.random.default_rng(31 * m + ncell)
+    ncell, n = len(trees), sum(len(t) for t in trees)
+    par, free = np.full(n, -1, np.int32), ncell
+    for c, t in enumerate(trees):
+        node = np.concatenate([[c], free + np.arange(len(t) - 1)]).astype(np.int64)
+        free += len(t) - 1
+        par[node[1:]] = node[np.asarray(t[1:], np.int64)]
+    rng = np.random.default_rng(31 * len(trees[0]) + ncell)
     a, b = -rng.uniform(0.05, 2.0, n), -rng.uniform(0.05, 2.0, n)
-    deg = np.bincount(par[ncell:], minlength=n) if m > 1 else np.zeros(n)
+    deg = np.bincount(par[ncell:], minlength=n) if n > ncell else np.zeros(n)
     a[ncell:] /= np.maximum(1.0, deg[par[ncell:]])
     a[:ncell] = b[:ncell] = 0.0
     mechs = {"pas": MechSpec(np.arange(n, dtype=np.int32),
@@ -101,6 +106,57 @@ def test_packs_change_no_bit(gpu_lib, unit_cells, groups):
     assert g.info("solve_split") == 1
     assert np.array_equal(base.traces(), g.traces())
     assert np.array_equal(base.get_array("global", "v"), g.get_array("global", "v"))
+
+
+# cells of about 3, 200, 400 and 620 chunks: a workgroup size each
+MIXED = [bushy(1000), bushy(330), bushy(640)] + [bushy(5), chain(3), bushy(330), chain(1), chain(20)]
+
+
+@pytest.mark.parametrize("clamp", [False, True])
+@pytest.mark.parametrize("small,unit_cells,launches", [(20, 1, 1), (600, 1, 4), (600, 3, 1), (2000, 3, 4)])
+def test_cells_of_unequal_size(gpu_lib, small, unit_cells, launches, clamp):
+    """One launch for all packs, padded to the largest, or one for each workgroup size."""
+    print(f"case split unequal small={small} unit_cells={unit_cells} clamp={clamp}", flush=True)
+    spec = forest(MIXED + [bushy(9)] * small, clamp)
+    s, r = run(spec, True, unit_cells=unit_cells), run(spec, False, unit_cells=unit_cells)
+    assert s.info("solve_split") == 1 and r.info("solve_split") == 0
+    assert s.info("solve_split_launches") == launches
+    assert float(np.max(np.abs(s.traces() - r.traces()))) < TOL
+    for k in ("v", "rhs"):
+        assert float(np.max(np.abs(s.get_array("global", k) - r.get_array("global", k)))) < TOL, k
+    np.testing.assert_allclose(s.get_array("global", "d"), r.get_array("global", "d"), rtol=TOL)
+    if unit_cells == 3:         # packs and classes change no bit
+        one = run(spec, True, unit_cells=1, groups=1 if clamp else 2)
+        assert np.array_equal(s.traces(), one.traces())
+        assert np.array_equal(s.get_array("global", "v"), one.get_array("global", "v"))
+    if small == 20:
+        o = oracle.OracleSim(spec, monitors=[("global", "v", c) for c in range(spec.ncell)])
+        o.finitialize(-65.0)
+        for _ in range(2):
+            o.continue_run(0.5)
+        assert float(np.max(np.abs(o.traces() - s.traces()))) < V_TOL
+
+
+def test_adjoint_of_cells_of_unequal_size(gpu_lib):
+    """The transposed solve, launch by launch, against the rounds; a gradient is a sum over
+    40 steps of terms that carry the solve's rounding (TOL, relative to the largest)."""
+    print("case split unequal adjoint", flush=True)
+    spec = forest(MIXED + [bushy(9)] * 600, True)
+    out = []
+    for split in (True, False):
+        g = Sim()
+        g.set_solve_unit_cells(1)
+        g.set_solve_split(split)
+        g.load_model_from_spec(spec, add_monitors=False)
+        g.tape_begin(40)
+        g.finitialize(-65.0)
+        g.run(40.25 * spec.dt)
+        assert g.info("solve_split_launches") == (4 if split else 0)
+        loss = g.adjoint(np.arange(spec.ncell), np.full((40, spec.ncell), -60.0))
+        out.append((loss, g.gradient("pas", "g_pas")))
+    assert abs(out[0][0] - out[1][0]) <= 1e-12 * abs(out[1][0])
+    scale = float(np.max(np.abs(out[1][1])))
+    assert scale > 0 and float(np.max(np.abs(out[0][1] - out[1][1]))) < TOL * scale
 
 
 def test_pivots_and_solution_on_demand(gpu_lib):
