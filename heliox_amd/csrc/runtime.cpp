@@ -4401,7 +4401,7 @@ int hx_set_fusion(hx_sim* sim, int enable) {
 
 int hx_set_group_turns(hx_sim* sim, int enable) {
     HX_SETTLE(sim);
-    sim->group_turns = enable ? 1 : 0;
+    sim->group_turns = enable < 0 ? -1 : enable ? 1 : 0;
     return 0;
 }
 
@@ -4669,8 +4669,8 @@ long long hx_get_info(hx_sim* sim, const char* key) {
     if (k == "solve_unit_cells") return sim->unit_cells;
     if (k == "solve_waves") return sim->solve_waves;
     if (k == "solve_resident") return sim->res_nodes > 0 ? 1 : 0;
-    if (k == "solve_split") return sim->solve_split ? 1 : 0;
-    if (k == "solve_split_launches") return sim->solve_split ? static_cast<long long>(sim->split_classes.size()) : 0;
+    if (k == "solve_split") return sim->use_split() ? 1 : 0;
+    if (k == "solve_split_launches") return sim->use_split() ? static_cast<long long>(sim->split_classes.size()) : 0;
     if (k == "solve_voltage") return sim->solve_voltage ? 1 : 0;
     if (k == "nchunk_total") return static_cast<long long>(sim->descs.size());
     if (k == "event_slots") return sim->groups.empty() ? 0 : sim->groups[0].ring.nslot;

@@ -328,10 +328,10 @@ class Sim:
     def set_fusion(self, enable: bool) -> int:
         return self._rc(lib().hx_set_fusion(self._h, 1 if enable else 0))
 
-    def set_group_turns(self, enable: bool) -> int:
-        """Make the cell groups' node passes take turns on every step (default on; same
-        results either way)."""
-        return self._rc(lib().hx_set_group_turns(self._h, 1 if enable else 0))
+    def set_group_turns(self, enable: Optional[bool]) -> int:
+        """Make the cell groups' node passes take turns on every step (None, the default: with
+        the round-by-round solve only; same results in any case)."""
+        return self._rc(lib().hx_set_group_turns(self._h, -1 if enable is None else int(bool(enable))))
 
     def set_dense_steady(self, enable: bool) -> int:
         """Run steady node-kernel steps through their compile-time instance (default on;

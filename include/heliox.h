@@ -328,8 +328,11 @@ int hx_set_solve_resident(hx_sim* sim, int enable);
  * ones).  0 solves round by round (hx_set_solve_resident), which also yields d and rhs after
  * a step in either case; a monitor, captured signal, transfer, optimizer or VecPlay entry
  * that names d or rhs runs both on every step.  The two agree to rounding: their voltages
- * differ in the last bits.  hx_get_info("solve_split") reports the choice (fixed at load)
- * and "solve_split_launches" the launches of a solve.  Call before hx_load_model. */
+ * differ in the last bits.  A taped run (hx_tape_begin) that solves for the new voltage
+ * (hx_set_solve_voltage) keeps the rounds, and so does its adjoint, so its voltages differ in
+ * the last bits from the same run's without a tape.  hx_get_info("solve_split") reports the
+ * route of the next steps, "solve_split_launches" the launches of a solve.  Call before
+ * hx_load_model. */
 int hx_set_solve_split(hx_sim* sim, int enable);
 /* Tree solve unknown (no counterpart in the reference): enable = 1 (default) lets a model
  * whose node kernel makes every term of d and rhs (no density mechanism on its own kernel,
@@ -342,10 +345,12 @@ int hx_set_solve_voltage(hx_sim* sim, int enable);
 /* Allow (1, default) or forbid (0) issuing the cell groups on their own streams in the
  * following runs; with 0 every launch goes to the library stream.  Same results. */
 int hx_set_group_streams(hx_sim* sim, int enable);
-/* No reference counterpart.  enable = 1 (default): with the cell groups on their own streams,
- * every step's node passes take turns (group g waits for group g-1's node pass, group 0 for the
- * last group's pass of the step before), so each group's tree solve runs beside the next group's
- * node pass; 0: only a run's first step is ordered that way.  Same results either way. */
+/* No reference counterpart.  enable = 1: with the cell groups on their own streams, every step's node
+ * passes take turns (group g waits for group g-1's node pass, group 0 for the last group's pass
+ * of the step before), so each group's tree solve runs beside the next group's node pass; 0:
+ * only a run's first step is ordered that way.  -1 (default): turns with the round-by-round
+ * solve, none with the solve by substructuring (hx_set_solve_split).  Same results in any
+ * case. */
 int hx_set_group_turns(hx_sim* sim, int enable);
 /* Layout facts: "nnode", "ncell", "nchunk_max", "nround_max", "dense_mask", "fused",
  * "cell_groups", "multi_stream" (1 if the last run used per-group streams), "state_pending"
@@ -355,7 +360,8 @@ int hx_set_group_turns(hx_sim* sim, int enable);
  * 16-23 parameter terms; bit 0 pas, 1 hh, 2 Ca_HVA, 3 hd_la, 4 CaDynamics_E2; bit 24: the synapses
  * too; bit 25: the loss term too), "steady_launches" (node-kernel launches so far that ran a
  * compile-time steady-step instance, see hx_set_dense_steady), "electrode_nodes" (nodes whose
- * IClamp and HalfGap currents one launch adds when the model has both). */
+ * IClamp and HalfGap currents one launch adds when the model has both), "solve_split" and
+ * "solve_split_launches" (hx_set_solve_split). */
 long long hx_get_info(hx_sim* sim, const char* key);
 
 /* ---- adjoint (VJP) backward pass: no reference counterpart.  It produces the
