@@ -346,6 +346,7 @@ struct hx_sim {
     bool need_dx = false, dx_pending = false;
     int dx_yform = 0;
     double* d_vold = nullptr;
+    bool rounds_last = false;            // the last step ran the rounds: its old voltages are in w
     // the packs of one workgroup size, one launch; those of unit u are
     // [unit_begin[u], unit_begin[u + 1])
     struct SplitClass {
@@ -2733,6 +2734,7 @@ SplitArgs hx_sim::split_args(const SplitClass& c, int unit0, int unit1) const {
 }
 
 void hx_sim::issue_solve(int unit0, int unit1, hipStream_t s) {
+    rounds_last = !use_split() || need_dx;
     if (!use_split()) {
         launch_solve(solve_args(unit0, unit1, store_dx()), max_slots, s);
         return;
@@ -3001,7 +3003,8 @@ bool hx_sim::lazy_outputs_ok() const {
 }
 
 // The node kernel's assigned outputs of the call's last step: its current evaluation
-// again, on the voltages before that step's solve (kept in w by k_solve<1>) and the
+// again, on the voltages before that step's solve (kept in w by the rounds, in d_vold by
+// k_solve_split, which the rounds beside it overwrite) and the
 // states it used (their update is still pending).  Its d and rhs go to w too (each
 // thread reads its own voltage there before it stores), so the solve's pivots and x
 // stay in d and rhs.
@@ -3013,7 +3016,7 @@ void hx_sim::launch_outputs_pass() {
     StepArgs A = step_args(t - 0.5 * dt, 0, 1);
     final_step = f;
     lazy_outputs_run = l;
-    A.v = solve_split ? d_vold : d_w;
+    A.v = rounds_last ? d_w : d_vold;
     A.d = d_w;
     A.rhs = d_w;
     A.fold_mask = 0;

@@ -200,6 +200,27 @@ def test_handles_and_monitors_of_the_solution(gpu_lib):
     assert np.array_equal(held.get_array("global", "d"), plain.get_array("global", "d"))
 
 
+def test_outputs_on_demand_after_a_reader_left(gpu_lib):
+    """A transfer that named rhs and is gone leaves the solution made on every step; the
+    outputs made later from the old voltages are the same run's without it."""
+    spec = build_config(3, 2, 2.0)
+    print("case split outputs after a transfer", flush=True)
+    out = []
+    for reader in (False, True):
+        g = Sim()
+        g.load_model_from_spec(spec)
+        if reader:
+            sid = g.add_gap_source(-1, "global", "rhs", 3)
+            assert sid >= 0 and g.add_gap_target(sid, "capacitance", "cm", 3) == 0
+            assert g.clear_all_gap_junctions() == 0
+        g.finitialize(-65.0)
+        g.continue_run(2.0)
+        assert g.info("solve_split") == 1 and g.info("outputs_pending") == 1
+        out.append([g.get_array(*k) for k in (("hh", "ina"), ("Ca_HVA", "ica"), ("pas", "i"), ("global", "v"))])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_vecplay_into_the_solution(gpu_lib):
     """VecPlay writes its rhs entry after each solve; the other entries stay the solution's."""
     spec = passive(bushy(60), 4, False)
