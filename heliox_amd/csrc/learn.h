@@ -172,7 +172,7 @@ void launch_rp_finish(ReplayFinishArgs a, hipStream_t s);
 int rp_finish_blocks(int N);
 void launch_rp_range(const ReplayRangeArgs& a, hipStream_t s);
 void launch_rp_tick(ReplayTickArgs a, hipStream_t s);
-void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s);
+void launch_rp_dx(const ReplayDx& a, int N, int corr_tile_cols, hipStream_t s);   // 0: k_rp_finish's sums
 void launch_rp_scale_into(const float* src, float scale, float* dst, long long n, hipStream_t s);
 void launch_fill_f32(float* p, float v, long long n, hipStream_t s);
 void launch_transpose_nt_tn(const float* src_nt, float* dst_tn, int N, int T, hipStream_t s);

@@ -157,9 +157,10 @@ __device__ __forceinline__ void rp_dx(const ReplayDx& X, int N, int j, float* sh
     if (tid == 0) row[X.t_idx] = st * bt;
 }
 
-__global__ void __launch_bounds__(kThreads) k_rp_dx(ReplayDx X, int N) {
-    __shared__ float sh[kThreads];
-    rp_dx<kThreads>(X, N, blockIdx.x, sh);
+template <int kT>
+__global__ void __launch_bounds__(kT) k_rp_dx(ReplayDx X, int N) {
+    __shared__ float sh[kT];
+    rp_dx<kT>(X, N, blockIdx.x, sh);
 }
 
 // ---------------------------------------------------------------- correction GEMM
@@ -636,8 +637,12 @@ void launch_rp_tick(ReplayTickArgs a, hipStream_t s) {
     else go(k_rp_tick<16, unsigned long long>, 16);
 }
 
-void launch_rp_dx(const ReplayDx& a, int N, hipStream_t s) {
-    if (a.n_in > 0) hipLaunchKernelGGL(k_rp_dx, dim3(a.n_in), dim3(kThreads), 0, s, a, N);
+// as k_rp_corr's blocks do it (their size sets the order of the sums) or as k_rp_finish's
+void launch_rp_dx(const ReplayDx& a, int N, int corr_tile_cols, hipStream_t s) {
+    if (a.n_in <= 0) return;
+    static_assert(CorrShape<128>::kT == 512 && CorrShape<64>::kT == 512 && CorrShape<32>::kT == kThreads);
+    if (corr_tile_cols >= 64) hipLaunchKernelGGL(k_rp_dx<512>, dim3(a.n_in), dim3(512), 0, s, a, N);
+    else hipLaunchKernelGGL(k_rp_dx<kThreads>, dim3(a.n_in), dim3(kThreads), 0, s, a, N);
 }
 
 void launch_rp_scale_into(const float* src, float scale, float* dst, long long n, hipStream_t s) {

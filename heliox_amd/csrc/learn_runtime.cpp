@@ -485,6 +485,16 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
             O.sanitize = due ? 1 : 0;
 
             const int nsplit = in.percise ? rp_corr_splits(N, ntiles, max_bnp_, tw) : 0;
+            // timed: the GEMM and the sum of its splits, with the previous tick's dx ahead of
+            // them (the same sums) instead of beside them
+            hipEvent_t ev[2] = {nullptr, nullptr};
+            if (timing) {
+                launch_rp_dx(X, N, nsplit == 1 ? tile_cols_ : 0, stream_);
+                X.n_in = 0;
+                for (auto& e : ev) LRC(hipEventCreate(&e));
+                evs.push_back({ev[0], ev[1]});
+                LRC(hipEventRecord(ev[0], stream_));
+            }
             if (in.percise) {
                 ReplayCorrArgs C{};
                 C.x = ws.x;
@@ -510,17 +520,7 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
                 C.part = ws.part;
                 C.O = O;
                 if (nsplit == 1) C.dx = X;
-                if (timing) {
-                    hipEvent_t a, b;
-                    LRC(hipEventCreate(&a));
-                    LRC(hipEventCreate(&b));
-                    LRC(hipEventRecord(a, stream_));
-                    launch_rp_corr(C, tile_cols_, stream_);
-                    LRC(hipEventRecord(b, stream_));
-                    evs.push_back({a, b});
-                } else {
-                    launch_rp_corr(C, tile_cols_, stream_);
-                }
+                launch_rp_corr(C, tile_cols_, stream_);
             }
             if (nsplit != 1) {
                 ReplayFinishArgs F{};
@@ -534,6 +534,7 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
                 F.dx = X;
                 launch_rp_finish(F, stream_);
             }
+            if (timing) LRC(hipEventRecord(ev[1], stream_));
             K.cur = O.out;
             K.due = due ? 1 : 0;
             K.npart = nsplit == 1 ? ntiles * row_tiles : rp_finish_blocks(N);
@@ -546,7 +547,7 @@ int LearnRuntime::replay_on(const ReplayIn& in, const Workspace& ws, float* cons
             X.t_idx = t_lr - 1;
             X.clip_ran = due ? 1 : 0;
         }
-        launch_rp_dx(X, N, stream_);
+        launch_rp_dx(X, N, 0, stream_);
         // dw = dw_accum * (1 / ksteps) in fp32 (LearnRuntime.cpp:2281-2285)
         launch_rp_scale_into(ws.dw_acc, 1.0f / static_cast<float>(ks), ws.dw_out, N, stream_);
         LRC(hipStreamSynchronize(stream_));

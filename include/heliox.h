@@ -487,8 +487,11 @@ int hx_simulate_and_replay_dw_dx_streaming_into(
     const int* didv_dest, const float* didv_scale, int n_didvpre, const int* didvpre_handles, const int* didvpre_dest,
     const float* didvpre_scale, double tstop_ms, int k_mul, int percise, double v_init, double dt_ms,
     double grad_scale, double eps, double grad_l2norm_threshold, int clip_strategy, int clip_check_every);
-/* Timing of the replay's correction-GEMM launches with HIP events on the library stream
- * (no counterpart in the reference; used by the benchmark). */
+/* Timing of the replay's correction with HIP events on the library stream (no counterpart in
+ * the reference; used by the benchmark): per tick, the correction GEMM with the sum of its
+ * splits (without the precise term, what makes the tick's slice).  While it is on, dx runs in
+ * launches of its own; results are the same.  ms is the total of the last replay, launches
+ * its ticks. */
 int hx_set_replay_timing(hx_sim* sim, int enable);
 int hx_get_replay_kernel_time(hx_sim* sim, double* ms, long long* launches);
 

@@ -42,6 +42,8 @@ CASES = [
     ((200, 199, 131), 2, 7, True, 0.3, False),
     ((128,) * 8 + (77,), 2, 5, True, 0.3, False),
     ((300,) * 7 + (1,), 2, 4, False, 0.3, False),
+    ((125,) * 12, 1, 3, True, 1e6, False),       # a tile for more than every other CU: no split
+    ((20,) * 70, 1, 3, True, 1e6, False),        # the same with 32-column tiles
 ]
 
 
@@ -68,6 +70,15 @@ def test_replay_at_tile_edges_matches_oracle(sim, bns, K_len, ksteps, percise, t
         rdw, rdx, _ = lrds.replay(it, dv, dp, blocks, dL, po, pre, dt=0.1, percise=percise, pinput=pin, grad_scale=1.3,
                                   eps=4.0, grad_l2norm_threshold=thr, clip_strategy=1, variant="signals")
     assert np.all(np.isfinite(rdw)) and np.all(np.isfinite(rdx))
+    # timed, dx runs apart from the correction: the same bits
+    dw2, dx2 = np.zeros_like(dw), np.zeros_like(dx)
+    sim.set_replay_timing(True)
+    rc = sim.replay_compute_dw_dx_from_signals_into(it, dv, dp, dL, po, pin, pre, dw2, dx2, 0.1, percise, grad_scale=1.3,
+                                                    eps=4.0, grad_l2norm_threshold=thr)
+    ms, ticks = sim.replay_kernel_time()
+    sim.set_replay_timing(False)
+    assert rc == 0 and ms > 0 and ticks == ksteps
+    assert np.array_equal(dw, dw2) and np.array_equal(dx, dx2)
     tol = 16 * np.sqrt(K_len * (max(bns) + 1)) * 2.0 ** -24
     for name, a, r in (("dw", dw, rdw), ("dx", dx, rdx)):
         err, scale = float(np.max(np.abs(a - r))), float(np.max(np.abs(r)))
