@@ -152,14 +152,16 @@ def perturb_config3(spec, seed: int = 1):
 
 
 def solver_options(sim, args):
-    """Tree-solve options of the command line (the layouts change no result; the two solve
-    forms agree to rounding)."""
+    """Tree-solve options of the command line (the layouts change no result; the solve's two
+    kernels and two forms agree to rounding)."""
     if args.unit_cells:
         sim.set_solve_unit_cells(args.unit_cells)
     if args.solve_waves:
         sim.set_solve_waves(args.solve_waves)
     if args.solve_streamed:
         sim.set_solve_resident(False)
+    if args.solve_rounds or args.solve_waves or args.solve_streamed:
+        sim.set_solve_split(False)
     if args.solve_change:
         sim.set_solve_voltage(False)
 
@@ -420,10 +422,14 @@ def main():
     ap.add_argument("--unit-cells", type=int, default=0,
                     help="cells per tree-solve wavefront (0: the library's choice)")
     ap.add_argument("--solve-waves", type=int, default=0,
-                    help="tree-solve wavefronts per workgroup (0: the library's choice)")
+                    help="tree-solve wavefronts per workgroup of the rounds (0: the library's choice; "
+                         "implies --solve-rounds)")
+    ap.add_argument("--solve-rounds", action="store_true",
+                    help="solve round by round, also where the solve by substructuring would be used "
+                         "(the two agree to rounding)")
     ap.add_argument("--solve-streamed", action="store_true",
                     help="stream every solve unit's rounds from HBM, also where the unit fits in LDS "
-                         "(same results)")
+                         "(same results as the rounds; implies --solve-rounds)")
     ap.add_argument("--solve-change", action="store_true",
                     help="solve for the change in voltage, as the reference does, also where the node "
                          "kernel makes every term of the matrix (the forms agree to rounding)")

@@ -20,9 +20,11 @@ def run(spec, resident, tstop, unit_cells=0, groups=1, chunks=2):
     g = Sim()
     g.set_cell_groups(groups)
     g.set_solve_unit_cells(unit_cells)
+    g.set_solve_split(False)          # the rounds themselves, on every step
     g.set_solve_resident(resident)
     mons = [("global", "v", c) for c in range(spec.ncell)]
     g.load_model_from_spec(dataclasses.replace(spec, monitors=mons))
+    assert g.info("solve_split") == 0
     g.finitialize(-65.0)
     for _ in range(chunks):
         g.continue_run(tstop / chunks)
@@ -84,9 +86,10 @@ def test_adjoint_transposed_solve_same_bits(gpu_lib):
     for resident in (True, False):
         print(f"case resident adjoint resident={resident}", flush=True)
         g = Sim()
+        g.set_solve_split(False)
         g.set_solve_resident(resident)
         g.load_model_from_spec(base, add_monitors=False)
-        assert g.info("solve_resident") == int(resident)
+        assert g.info("solve_resident") == int(resident) and g.info("solve_split") == 0
         g.tape_begin(target.shape[0])
         g.finitialize(-65.0)
         g.run(tstop)

@@ -1,8 +1,8 @@
 """The solve for the new voltage (the node kernel stores rhs + d v, the solve never reads v)
 against the reference's solve for the change x = v_new - v: both against the oracle to the
 voltage tolerance and to each other to rounding, with one cell group and with cell groups
-on their own streams, through the resident and the streamed solve; rhs holds x after a
-call either way; models where a later kernel adds to d or rhs keep the reference's form."""
+on their own streams, through the resident and the streamed rounds and the solve by
+substructuring; rhs holds x after a call either way; models where a later kernel adds to d or rhs keep the reference's form."""
 import dataclasses
 
 import numpy as np
@@ -37,13 +37,15 @@ def model(config, ncell, tstop):
     return hh_everywhere(build_config(5, ncell, tstop)) if config == "5hh" else build_config(config, ncell, tstop)
 
 
-def run(spec, voltage, tstop, groups=1, resident=True):
+def run(spec, voltage, tstop, groups=1, resident=True, split=True):
     g = Sim()
+    g.set_solve_split(split)
     g.set_cell_groups(groups)
     g.set_solve_resident(resident)
     g.set_solve_voltage(voltage)
     mons = [("global", "v", c) for c in range(spec.ncell)]
     g.load_model_from_spec(dataclasses.replace(spec, monitors=mons))
+    assert g.info("solve_split") == int(split)
     g.finitialize(-65.0)
     g.continue_run(tstop / 2)     # a duration
     g.continue_run(tstop / 2)
@@ -58,14 +60,16 @@ def oracle_traces(spec, tstop):
     return o
 
 
-@pytest.mark.parametrize("config,ncell,tstop,groups,resident", [
-    (3, 2, 10.0, 1, True), (3, 16, 4.0, 2, True), ("5hh", 8, 20.0, 1, True), ("5hh", 24, 20.0, 2, True),
-    ("5hh", 8, 20.0, 1, False)])
-def test_voltage_form_matches_the_change_form(gpu_lib, config, ncell, tstop, groups, resident):
+@pytest.mark.parametrize("config,ncell,tstop,groups,resident,split", [
+    (3, 2, 10.0, 1, True, False), (3, 16, 4.0, 2, True, False), ("5hh", 8, 20.0, 1, True, False),
+    ("5hh", 24, 20.0, 2, True, False), ("5hh", 8, 20.0, 1, False, False),
+    (3, 2, 10.0, 1, True, True), (3, 16, 4.0, 2, True, True), ("5hh", 24, 20.0, 2, True, True)])
+def test_voltage_form_matches_the_change_form(gpu_lib, config, ncell, tstop, groups, resident, split):
     spec = model(config, ncell, tstop)
-    print(f"case solve voltage config={config} ncell={ncell} groups={groups} resident={resident}", flush=True)
-    y = run(spec, True, tstop, groups, resident)
-    x = run(spec, False, tstop, groups, resident)
+    print(f"case solve voltage config={config} ncell={ncell} groups={groups} resident={resident} split={split}",
+          flush=True)
+    y = run(spec, True, tstop, groups, resident, split)
+    x = run(spec, False, tstop, groups, resident, split)
     assert y.info("solve_voltage") == 1
     assert x.info("solve_voltage") == 0
     assert y.info("cell_groups") == groups

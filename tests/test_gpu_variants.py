@@ -19,8 +19,9 @@ from parity_util import V_TOL, compare_spikes, run_both
 pytestmark = pytest.mark.gpu
 
 
-def run(spec, steady, chunks=(5.0,), groups=1, mons=None, fusion=True, turns=True):
+def run(spec, steady, chunks=(5.0,), groups=1, mons=None, fusion=True, turns=True, split=True):
     g = Sim()
+    g.set_solve_split(split)
     g.set_cell_groups(groups)
     g.load_model_from_spec(spec if mons is None else dataclasses.replace(spec, monitors=list(mons)))
     g.set_dense_steady(steady)
@@ -96,15 +97,18 @@ def test_no_steady_instance_when_fusion_is_off_or_an_output_is_sampled(gpu_lib):
     same_everything(spec, b, c)
 
 
+@pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("groups", [2, 3])
-def test_group_turns_same_bits(gpu_lib, groups):
+def test_group_turns_same_bits(gpu_lib, groups, split):
     # groups hold at least 8 cells each
     spec = build_config(3, 8 * groups, 6.0)
-    print(f"case group turns, config 3, {groups} groups", flush=True)
-    a = run(spec, True, chunks=(1.0, 2.5, 0.5), groups=groups, turns=True)
-    b = run(spec, True, chunks=(1.0, 2.5, 0.5), groups=groups, turns=False)
+    print(f"case group turns, config 3, {groups} groups, split={split}", flush=True)
+    a = run(spec, True, chunks=(1.0, 2.5, 0.5), groups=groups, turns=True, split=split)
     assert a.info("cell_groups") == groups and a.info("multi_stream") == 1
-    same_everything(spec, a, b)
+    assert a.info("solve_split") == int(split)
+    for turns in (False, None):
+        b = run(spec, True, chunks=(1.0, 2.5, 0.5), groups=groups, turns=turns, split=split)
+        same_everything(spec, a, b)
 
 
 def test_iclamp_and_halfgap_in_one_launch(gpu_lib):
