@@ -319,8 +319,6 @@ int LearnRuntime::replay(const ReplayIn& in) {
             ws_.slices = lalloc<float>(ws_mem_, 2 * slice);
             ws_.x = lalloc<float>(ws_mem_, z.x);
             ws_.part = lalloc<float>(ws_mem_, z.part);
-            ws_.base_ticks = kBaseTicks;
-            ws_.base = lalloc<float>(ws_mem_, static_cast<size_t>(base_len_) * kBaseTicks);
             ws_.xscale = lalloc<float>(ws_mem_, z.xscale);
             ws_.xdown = lalloc<unsigned char>(ws_mem_, z.xscale ? static_cast<size_t>(ks) * xcols_ / 4 : 0);
             ws_.gs = lalloc<float>(ws_mem_, 1);
@@ -334,11 +332,26 @@ int LearnRuntime::replay(const ReplayIn& in) {
             ws_.dx = lalloc<float>(ws_mem_, static_cast<size_t>(std::max(in.n_in, 1)) * ks);
             ws_.norm_part = lalloc<double>(ws_mem_, z.norm);
             ws_.dw_out = lalloc<float>(ws_mem_, N);
+            // the base terms of as many ticks as there is memory for (one block's are N^2 floats
+            // a tick; how many are made at a time changes no result)
+            ws_.base = nullptr;
+            for (ws_.base_ticks = kBaseTicks; !ws_.base; ws_.base_ticks /= 2) {
+                void* p = nullptr;
+                const size_t bytes = sizeof(float) * static_cast<size_t>(base_len_) * ws_.base_ticks;
+                if (hipMalloc(&p, bytes) == hipSuccess) {
+                    ws_mem_.push_back(p);
+                    ws_.base = static_cast<float*>(p);
+                    break;
+                }
+                (void)hipGetLastError();
+                if (ws_.base_ticks == 1) throw HipFail("out of device memory for the base term");
+            }
             // the padding of the X rows stays zero: only the columns themselves are written
             if (z.x) launch_fill_f32(ws_.x, 0.f, static_cast<long long>(z.x), stream_);
             ws_key_ = key;
         }
     } catch (const std::exception& e) {
+        (void)hipGetLastError();          // not the next call's
         free_all(ws_mem_);
         ws_key_.clear();
         return fail("replay: %s", e.what());

@@ -84,3 +84,33 @@ def test_replay_at_tile_edges_matches_oracle(sim, bns, K_len, ksteps, percise, t
         err, scale = float(np.max(np.abs(a - r))), float(np.max(np.abs(r)))
         print(f"  {name} max err {err:.3e} scale {scale:.3e} tol {tol:.1e}", flush=True)
         assert err <= tol * scale + 1e-9
+
+
+def test_base_term_of_fewer_ticks_where_memory_is_short(gpu_lib):
+    """One block of 4000 columns: a tick's base terms are 64 MB, eight ticks' 512; with about
+    700 MB free the replay (448 MB beside them) makes fewer at a time, and the same bits."""
+    import torch
+
+    print("case lrds base ticks in short memory", flush=True)
+    rng = np.random.default_rng(4)
+    N, ksteps = 4000, 9
+    block = (rng.standard_normal((N, N, 1), np.float32) * np.float32(0.3 / np.sqrt(N)))
+    it, dv, dp = (rng.normal(0, 0.3, (N, ksteps + 1)).astype(np.float32) for _ in range(3))
+    pre = rng.integers(-1, N, N).astype(np.int32)
+    po, pin = np.arange(0, N, 500, dtype=np.int32), np.array([3], np.int32)
+    dL = rng.normal(0, 1, (ksteps, po.size)).astype(np.float32)
+    out = []
+    for short in (False, True):
+        g = Sim()
+        g.load_model_from_spec(build_config(1, 1, 10.0))
+        torch.cuda.empty_cache()
+        hold = torch.empty(torch.cuda.mem_get_info()[0] - (700 << 20), dtype=torch.uint8, device="cuda") if short else None
+        dw, dx = np.zeros(N, np.float32), np.zeros((1, ksteps), np.float32)
+        assert g.set_dense_blocks_f32([block]) == 1
+        rc = g.replay_compute_dw_dx_from_signals_into(it, dv, dp, dL, po, pin, pre, dw, dx, 0.1, True, eps=4.0)
+        assert rc == 0, g.last_error()
+        g.clear_dense_blocks()
+        del hold
+        torch.cuda.empty_cache()
+        out.append((dw, dx))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]) and np.any(out[0][0])
