@@ -1273,7 +1273,8 @@ __global__ void __launch_bounds__(kWave * kSolveMaxWaves) k_solve_res(SolveArgs 
 //   x_k = u_k - w_k x_{k+1} - f_k x_p.
 // The serial chain is one chunk plus a short step per level instead of a whole chunk per
 // round, and u, w and f stay in registers: a node is read once (d, rhs, a, b, v) and
-// written once (v), 48 bytes (40 with kY) where the streamed rounds move 80 (72).
+// written once (v), and without kY v is read again for the write, 56 bytes (40 with kY)
+// where the streamed rounds move 80 (72).
 // Which unit or pack a cell sits in changes no arithmetic, so the bits do not depend on it.
 // d and rhs keep the assembled matrix; the pivots and x that the reference leaves there
 // come from the round-by-round solve when something reads them.  Bound by latency: the dependent loads
@@ -1294,8 +1295,9 @@ inline size_t split_lds_bytes(int threads, int lev_stride) {
     return static_cast<size_t>(threads) * (sizeof(double) * (kSplitFields + 1) + 2 * sizeof(int)) +
            sizeof(int) * lev_stride;
 }
-// kT: the largest workgroup.  Up to 512 threads nothing spills; the change form at 768 (168
-// registers a thread) spills 34 of them, the voltage form none.
+// kT: the largest workgroup.  Up to 512 threads nothing spills (157 registers with kY, 12
+// wavefronts a CU; 184 without, 8); the change form at 768 (168 registers, 12 wavefronts)
+// spills 34 of them, the voltage form none.
 template <int kX, int kY, int kT>
 __global__ void __launch_bounds__(kT) k_solve_split(SplitArgs S) {
     extern __shared__ double lds[];

@@ -174,9 +174,9 @@ __global__ void __launch_bounds__(kT) k_rp_dx(ReplayDx X, int N) {
 // wave's ds_read_b128 over all banks.  Each such read feeds four MFMAs: which of the four
 // k a step takes is the same for both operands.
 // Bound: the fp32 matrix cores (157 TFLOP/s; a library product of 8192^3 reaches 153).
-// N = 2048 in 16 blocks of 128, K_len 64: 630 -> 439 us a launch over 128 ticks, 118
-// TFLOP/s with the window full (before: X formed while staging from two history rings, one
-// element per load).  Chunks of 32 with two workgroups per CU: 3% slower.
+// N = 2048 in 16 blocks of 128, K_len 64, 256 ticks: 725 -> 508 us a launch, 118.7 TFLOP/s
+// (before: X formed while staging from two history rings, one element per load).  Chunks of
+// 32 with two workgroups per CU: 3% slower.
 constexpr int kTI = 128;
 constexpr int kKC = 64;
 constexpr int kLd = kKC + 4;
@@ -348,11 +348,11 @@ __device__ __forceinline__ void next_element(I N, I& row, I& col) {
 
 // The tick's slice from the correction's split sums, added in split order (nsplit 0: no
 // correction), kE elements per thread; the previous tick's dx on blocks of its own.  The
-// splits are read four at a time, so a thread has 4 kE loads in flight (one at a time,
-// waiting for each, the kernel took 52 us at N = 400 with 28 splits); so are the block
-// look-ups of a thread's columns (a division, a look-up and a store one element after the
-// other: 4.2 ms at N = 32768 without splits, now 1.4; 4.3 GB written take 0.85).  I indexes the N x N
-// elements: unsigned, or 64 bits from about N = 65400.
+// splits are read four at a time, so a thread has 4 kE loads in flight (5.2 us at N = 400
+// with 16 splits); the block look-ups of a thread's columns are in flight together too (a
+// division, a look-up and a store one element after the other: 4.2 ms at N = 32768 without
+// splits, now 1.4; the 4.3 GB written take 0.85).  I indexes the N x N elements: unsigned,
+// or 64 bits from about N = 65400.
 template <int kE, class I>
 __global__ void __launch_bounds__(kThreads) k_rp_finish(ReplayFinishArgs A) {
     __shared__ double sh[kThreads];
@@ -483,6 +483,9 @@ __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
         }
         return;
     }
+    // the exponent is asked for ahead of the norm: its latency would follow the sum's
+    const int g0 = blockIdx.x * kThreads + tid;
+    const int down0 = A.x && g0 < A.xgroups ? A.xdown[g0] : 0;
     float sc = 1.f;
     if (A.due) {
         double acc = 0.0;
@@ -497,12 +500,11 @@ __global__ void __launch_bounds__(kThreads) k_rp_tick(ReplayTickArgs A) {
         }
     }
     if (A.x) {                                                // the scales of X's groups
-        const int first = sc != 1.f ? 0 : A.cur_slot, last = sc != 1.f ? A.R : A.cur_slot + 1;
-        const int here = A.cur_slot * A.xgroups;
-        for (int q = first * A.xgroups + blockIdx.x * kThreads + tid; q < last * A.xgroups; q += A.wblocks * kThreads) {
-            const int g = q - here;
-            A.xscale[q] = g >= 0 && g < A.xgroups ? ldexpf(sc, A.xdown[g]) : A.xscale[q] * sc;
-        }
+        const int here = A.cur_slot * A.xgroups, stride = A.wblocks * kThreads;
+        for (int g = g0; g < A.xgroups; g += stride) A.xscale[here + g] = ldexpf(sc, g == g0 ? down0 : A.xdown[g]);
+        if (sc != 1.f)
+            for (int q = g0; q < A.R * A.xgroups; q += stride)
+                if (q < here || q >= here + A.xgroups) A.xscale[q] *= sc;
     }
     const unsigned row = blockIdx.x * (kThreads / 64) + (tid >> 6);
     const int lane = tid & 63;

@@ -89,7 +89,7 @@ def test_replay_at_tile_edges_matches_oracle(sim, bns, K_len, ksteps, percise, t
 def test_base_term_of_fewer_ticks_where_memory_is_short(gpu_lib):
     """One block of 4000 columns: a tick's base terms are 64 MB, eight ticks' 512; with about
     700 MB free the replay (448 MB beside them) makes fewer at a time, and the same bits."""
-    import torch
+    import ctypes as C
 
     print("case lrds base ticks in short memory", flush=True)
     rng = np.random.default_rng(4)
@@ -103,14 +103,51 @@ def test_base_term_of_fewer_ticks_where_memory_is_short(gpu_lib):
     for short in (False, True):
         g = Sim()
         g.load_model_from_spec(build_config(1, 1, 10.0))
-        torch.cuda.empty_cache()
-        hold = torch.empty(torch.cuda.mem_get_info()[0] - (700 << 20), dtype=torch.uint8, device="cuda") if short else None
+        with open("/proc/self/maps") as f:      # the runtime that the library runs on
+            paths = {line.split()[-1] for line in f if "libamdhip64" in line}
+        hip = C.CDLL(sorted(paths, key=lambda p: "torch" in p)[0])
+        hold, free, total = C.c_void_p(), C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        if short:
+            assert hip.hipMalloc(C.byref(hold), C.c_size_t(free.value - (700 << 20))) == 0
         dw, dx = np.zeros(N, np.float32), np.zeros((1, ksteps), np.float32)
         assert g.set_dense_blocks_f32([block]) == 1
         rc = g.replay_compute_dw_dx_from_signals_into(it, dv, dp, dL, po, pin, pre, dw, dx, 0.1, True, eps=4.0)
-        assert rc == 0, g.last_error()
+        why = g.last_error()
         g.clear_dense_blocks()
-        del hold
-        torch.cuda.empty_cache()
+        if short:
+            assert hip.hipFree(hold) == 0
+        assert rc == 0, why
         out.append((dw, dx))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]) and np.any(out[0][0])
+
+
+def test_signal_buffers_serve_problems_of_other_sizes(gpu_lib):
+    """One program replays problems of growing and shrinking sizes, with and without the
+    precise term; each gives a fresh program's bits."""
+    print("case lrds signal buffers", flush=True)
+    rng = np.random.default_rng(8)
+    kept = Sim()
+    kept.load_model_from_spec(build_config(1, 1, 10.0))
+    blocks, last = None, 0
+    for n, ksteps, percise in [(40, 6, True), (40, 30, False), (200, 30, False), (200, 29, True), (40, 6, True),
+                               (12, 4, False), (12, 5, True), (12, 60, True)]:
+        if n != last:
+            blocks, last = [(rng.normal(0, 0.1, (n // 2, n // 2, 3))).astype(np.float32) for _ in range(2)], n
+            assert kept.set_dense_blocks_f32(blocks) == 3
+        it, dv, dp = (rng.normal(0, 0.5, (n, ksteps + 1)).astype(np.float32) for _ in range(3))
+        pre = rng.integers(-1, n, n).astype(np.int32)
+        dL = rng.normal(0, 1, (ksteps, 2)).astype(np.float32)
+        fresh = Sim()
+        fresh.load_model_from_spec(build_config(1, 1, 10.0))
+        assert fresh.set_dense_blocks_f32(blocks) == 3
+        out = []
+        for g in (kept, fresh):
+            dw, dx = np.zeros(n, np.float32), np.zeros((2, ksteps), np.float32)
+            rc = g.replay_compute_dw_dx_from_signals_into(it, dv, dp, dL, np.array([0, n - 1], np.int32),
+                                                          np.array([1, 2], np.int32), pre, dw, dx, 0.1, percise, eps=4.0,
+                                                          grad_l2norm_threshold=0.05)
+            assert rc == 0, g.last_error()
+            out.append((dw, dx))
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]), (n, ksteps, percise)
+        assert np.any(out[0][0])
