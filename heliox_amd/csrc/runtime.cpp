@@ -1056,10 +1056,11 @@ void hx_sim::build_layout() {
 // the chip holds at once (256 CUs; 12 wavefronts of the voltage form's 157 registers, 8 of
 // the change form's 184, 12 of its 768-thread instance).  A launch of more than a pass has
 // workgroups queueing, and the rounds, which leave room for the other group's node pass
-// beside them, catch up: at one pass where something couples the cells (one group, one
+// beside them, catch up: at 1.05 where something couples the cells (one group, one
 // launch), at 1.7 otherwise (two groups), and one later where the rounds are streamed from
 // HBM (87 us a step for 5000-node cells).  us a step, split and rounds:
 //   one group, change form: 12000 101-node cells (0.82 passes) 33, 40; 16000 (1.1) 53, 43;
+//     2500 500-node cells (1.04) 44, 67; 3000 (1.24) 64, 53;
 //     200-node network, 6000 cells (0.96) 72, 77; 8000 (1.3) 101, 88;
 //   two groups, change form: 4000 500-node cells (1.64) 86, 92; 5000 (2.05) 118, 97;
 //   two groups, voltage form: 5000 500-node cells (1.38) 60, 68; 6500 (1.8) 75, 70;
@@ -1147,7 +1148,7 @@ void hx_sim::build_packs() {
     }
     const bool resident_cells = static_cast<size_t>(max_nodes) * kStageArrays * sizeof(double) <= kResUnitBudget;
     solve_split = solve_split_allowed && !packs.empty() &&
-                  passes <= (groups_coupled ? 1.0 : 1.7) + (resident_cells ? 0.0 : 1.0);
+                  passes <= (groups_coupled ? 1.05 : 1.7) + (resident_cells ? 0.0 : 1.0);
     if (!solve_split) return;
     // A launch has one workgroup size.  One launch for all packs while they run in two
     // passes of the largest (1 pyramidal cell beside 200 101-node cells: 39 us a step, 47
